@@ -15,6 +15,7 @@
 
 #include "common.h"
 #include "w4a16_gemm_sk.h"
+#include "w4a16_rows.h"
 
 namespace mcv {
 
@@ -22,9 +23,7 @@ int launch_w4a16_gemv(const void* x, int64_t M, int64_t K, int64_t N, const void
                       const void* zeros, int zero_bias, void* out, hipStream_t stream);
 int gemv_ksplit(int64_t G, int64_t blocks);
 
-namespace {
-
-// Few rows: the GEMV streams the weights once per row and still beats the
+// The few-row kernels aside (w4a16_rows_pays comes first): the GEMV streams the weights once per row and still beats the
 // MFMA GEMM, whose tile count is M/TM * N/TN, until the output reaches about
 // 64K elements (MI355X, rotated weights: K=1024 N=3584 M=16 5.7 us against
 // 7.0; K=3584 N=1024 M=48 12.4 against 12.5; K=1024 N=6144 crosses over near
@@ -98,6 +97,20 @@ SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split) {
     return finish(c);
 }
 
+namespace {
+
+// The GEMV or (through launch_w4a16_gemv) the few-row kernels take this call.
+// The few-row kernels need an aligned x and 32-bit offsets; a call without them
+// goes where it always went.
+bool takes_gemv(const void* x, int64_t M, int64_t K, int64_t N) {
+    if (w4a16_prefers_gemv(M, N)) return true;
+    if (x == nullptr || M < 2 || K <= 0 || K % kGroup != 0 || N <= 0 || N > (int64_t(1) << 30)) return false;
+    W4Parts parts{};
+    parts.count = 1;
+    parts.p[0].Npad = static_cast<int>(ceil_div(N, kSlab) * kSlab);
+    return w4a16_rows_pays(M, K, ceil_div(N, kSlab), 1) && w4a16_rows_ok(x, M, K, parts);
+}
+
 int check_gemm_args(const void* x, int64_t M, int64_t K, int64_t N, const void* qw, const void* scales,
                     const void* zeros, int zero_bias, const void* out, const char* who) {
     if (!x || !out || !qw || !scales || !zeros) return fail(MCV_ERR_INVALID_ARG, "%s: null pointer", who);
@@ -140,7 +153,9 @@ int mcv_w4a16_gemm_mfma(const void* x, int64_t M, int64_t K, int64_t N, const vo
 }
 
 int64_t mcv_w4a16_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N) {
-    if (M < 1 || K <= 0 || N <= 0 || K % kGroup != 0 || w4a16_prefers_gemv(M, N)) return 0;
+    if (M < 1 || K <= 0 || N <= 0 || K % kGroup != 0 || w4a16_prefers_gemv(M, N) ||
+        w4a16_rows_pays(M, K, ceil_div(N, kSlab), 1))
+        return 0;
     return w4a16_sk_workspace_bytes(M, N, choose_gemm(M, K, N, true));
 }
 
@@ -149,7 +164,7 @@ int64_t mcv_w4a16_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N) {
 int mcv_w4a16_gemm_ws(const void* x, int64_t M, int64_t K, int64_t N, const void* qw, const void* scales,
                       const void* zeros, int zero_bias, void* out, void* workspace, int64_t workspace_bytes,
                       mcv_stream_t stream) {
-    if (w4a16_prefers_gemv(M, N))
+    if (takes_gemv(x, M, K, N))
         return launch_w4a16_gemv(x, M, K, N, qw, scales, zeros, zero_bias, out, static_cast<hipStream_t>(stream));
     return launch_w4a16_gemm_mfma(x, M, K, N, qw, scales, zeros, zero_bias, out, static_cast<hipStream_t>(stream),
                                   workspace, workspace_bytes);
@@ -159,7 +174,7 @@ int mcv_w4a16_gemm_ws(const void* x, int64_t M, int64_t K, int64_t N, const void
 // goes to the MFMA kernel, which reuses each dequantised operand across rows.
 int mcv_w4a16_gemm(const void* x, int64_t M, int64_t K, int64_t N, const void* qw, const void* scales,
                    const void* zeros, int zero_bias, void* out, mcv_stream_t stream) {
-    if (w4a16_prefers_gemv(M, N))
+    if (takes_gemv(x, M, K, N))
         return launch_w4a16_gemv(x, M, K, N, qw, scales, zeros, zero_bias, out, static_cast<hipStream_t>(stream));
     return launch_w4a16_gemm_mfma(x, M, K, N, qw, scales, zeros, zero_bias, out, static_cast<hipStream_t>(stream),
                                   nullptr, 0);
@@ -169,6 +184,8 @@ const char* mcv_w4a16_gemm_kernel_name(int64_t M, int64_t K, int64_t N, int with
     char buf[160];
     if (M < 1 || K <= 0 || N <= 0 || K % kGroup != 0) {
         g_kernel_name = "none (bad shape)";
+    } else if (w4a16_rows_pays(M, K, ceil_div(N, kSlab), 1)) {
+        g_kernel_name = w4a16_rows_name(M, K, ceil_div(N, kSlab));
     } else if (w4a16_prefers_gemv(M, N)) {
         std::snprintf(buf, sizeof(buf), "w4a16_gemv_kernel<%d, 1, 0> (grid %lld x %lld)",
                       gemv_ksplit(K / kGroup, ceil_div(N, kSlab) * M), (long long)ceil_div(N, kSlab), (long long)M);

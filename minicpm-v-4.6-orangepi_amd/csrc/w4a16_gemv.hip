@@ -22,6 +22,7 @@
 #include "argmax_exchange.h"
 #include "common.h"
 #include "gemv_body.h"
+#include "w4a16_rows.h"
 
 namespace mcv {
 namespace {
@@ -239,24 +240,8 @@ __global__ __launch_bounds__(64 * kLmWaves) void w4a16_lm_head_kernel(
 // weight from the running slab ends and then does exactly what the GEMV above
 // does with GPW = 1, so with the same k-split the outputs are bit-identical to
 // separate launches.
-constexpr int kMaxParts = 4;
-struct GemvPart {
-    const uint4* qw;
-    const uint16_t* scales;
-    const uint32_t* zeros;
-    uint16_t* out;
-    int N;
-    int Npad;
-    int slab_end;          // running total of slabs up to and including this part
-    uint32_t zero_bias;
-};
-struct GemvParts {
-    GemvPart p[kMaxParts];
-    int count;
-};
-
 template <int KSPLIT>
-__global__ __launch_bounds__(64 * KSPLIT) void w4a16_gemv_multi_kernel(const uint16_t* __restrict__ x, GemvParts parts,
+__global__ __launch_bounds__(64 * KSPLIT) void w4a16_gemv_multi_kernel(const uint16_t* __restrict__ x, W4Parts parts,
                                                                         int K) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -264,13 +249,13 @@ __global__ __launch_bounds__(64 * KSPLIT) void w4a16_gemv_multi_kernel(const uin
     const int m = blockIdx.y;
     // the part this slab belongs to (constant indices only: the kernel
     // arguments stay in SGPRs)
-    GemvPart P = parts.p[0];
+    W4Part P = parts.p[0];
     int slab0 = 0;
 #pragma unroll
     for (int j = 1; j < kMaxParts; ++j) {
-        if (j < parts.count && gslab >= parts.p[j - 1].slab_end) {
+        if (j < parts.count && gslab >= parts.p[j - 1].end) {
             P = parts.p[j];
-            slab0 = parts.p[j - 1].slab_end;
+            slab0 = parts.p[j - 1].end;
         }
     }
     const int slab = gslab - slab0;
@@ -588,6 +573,16 @@ static __device__ __align__(256) unsigned long long scratch[kNoallocWords];
 
 }  // namespace
 
+namespace {
+
+W4Part w4_part(const void* qw, const void* scales, const void* zeros, int zero_bias, int64_t N, void* out) {
+    return W4Part{static_cast<const uint4*>(qw), static_cast<const uint16_t*>(scales), static_cast<const uint32_t*>(zeros),
+                  static_cast<uint16_t*>(out), static_cast<int>(N), static_cast<int>(ceil_div(N, kSlab) * kSlab), 0,
+                  static_cast<uint32_t>(zero_bias)};
+}
+
+}  // namespace
+
 // The GEMV launchers' k-split, for kernels that must add in the same order
 // (decode_mlp.hip).
 int gemv_ksplit(int64_t G, int64_t blocks) { return choose_gemv(G, blocks).ksplit; }
@@ -601,6 +596,10 @@ int launch_w4a16_gemv(const void* x, int64_t M, int64_t K, int64_t N, const void
     if (M <= 0 || M > 65535) return fail(MCV_ERR_SHAPE, "mcv_w4a16_gemv: M must be in [1, 65535] (M=%lld)", (long long)M);
     if ((rc = require_device()) != MCV_OK) return rc;
     const int64_t nslab = ceil_div(N, kSlab);
+    W4Parts parts{};
+    parts.count = 1;
+    parts.p[0] = w4_part(qw, scales, zeros, zero_bias, N, out);
+    if (w4a16_rows_pays(M, K, nslab, 1) && w4a16_rows_ok(x, M, K, parts)) return launch_w4a16_rows(x, M, K, parts, stream);
     const GemvCfg cfg = choose_gemv(K / kGroup, nslab * M);
     auto fn = pick_kernel<kArgNone>(cfg.ksplit, cfg.gpw);
     hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(nslab), static_cast<unsigned>(M)), dim3(64 * cfg.ksplit), 0,
@@ -829,7 +828,7 @@ int mcv_w4a16_gemv_multi(const void* x, int64_t M, int64_t K, const mcv_w4a16_pa
     if (n_parts < 1 || n_parts > kMaxParts)
         return fail(MCV_ERR_INVALID_ARG, "mcv_w4a16_gemv_multi: 1..%d parts (got %d)", kMaxParts, n_parts);
     if (M <= 0 || M > 65535) return fail(MCV_ERR_SHAPE, "mcv_w4a16_gemv_multi: M must be in [1, 65535] (M=%lld)", (long long)M);
-    GemvParts gp{};
+    W4Parts gp{};
     int64_t total = 0;
     int64_t min_slabs = INT64_MAX;
     for (int i = 0; i < n_parts; ++i) {
@@ -841,19 +840,20 @@ int mcv_w4a16_gemv_multi(const void* x, int64_t M, int64_t K, const mcv_w4a16_pa
         total += ns;
         min_slabs = ns < min_slabs ? ns : min_slabs;
         if (total > 0x7fffffff) return fail(MCV_ERR_SHAPE, "mcv_w4a16_gemv_multi: too many columns");
-        gp.p[i] = GemvPart{static_cast<const uint4*>(q.qw_dev), static_cast<const uint16_t*>(q.scales_dev),
-                           static_cast<const uint32_t*>(q.zeros_dev), static_cast<uint16_t*>(q.out_dev),
-                           static_cast<int>(q.N), static_cast<int>(ns * kSlab), static_cast<int>(total),
-                           static_cast<uint32_t>(q.zero_bias)};
+        gp.p[i] = w4_part(q.qw_dev, q.scales_dev, q.zeros_dev, q.zero_bias, q.N, q.out_dev);
+        gp.p[i].end = static_cast<int>(total);
     }
     gp.count = n_parts;
     int rc = require_device();
     if (rc != MCV_OK) return rc;
+    // a few rows: each weight widened once for all of them
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    if (w4a16_rows_pays(M, K, total, n_parts) && w4a16_rows_ok(x, M, K, gp)) return launch_w4a16_rows(x, M, K, gp, st);
     // The k-split the smallest part would get on its own (the decode shapes
     // with K = 1024 all get 8, so the outputs equal separate launches').
     const GemvCfg cfg = choose_gemv(K / kGroup, min_slabs * M);
     const int ks = cfg.ksplit;
-    using Fn = void (*)(const uint16_t*, GemvParts, int);
+    using Fn = void (*)(const uint16_t*, W4Parts, int);
     Fn fn = ks >= 16 ? w4a16_gemv_multi_kernel<16>
           : ks == 8 ? w4a16_gemv_multi_kernel<8>
           : ks == 4 ? w4a16_gemv_multi_kernel<4>
@@ -875,6 +875,14 @@ int mcv_w4a16_gate_up_silu(const void* x, int64_t M, int64_t K, int64_t N, const
     if (M <= 0 || M > 65535) return fail(MCV_ERR_SHAPE, "mcv_w4a16_gate_up_silu: M must be in [1, 65535] (M=%lld)", (long long)M);
     if ((rc = require_device()) != MCV_OK) return rc;
     const int64_t nslab = ceil_div(N, kSlab);
+    // a few rows as in mcv_w4a16_gemv_multi; the rule is the single weight's, so gate and up round as two mcv_w4a16_gemv calls do
+    W4Parts parts{};
+    parts.count = 2;
+    parts.p[0] = w4_part(qw_gate, scales_gate, zeros_gate, zero_bias_gate, N, act);
+    parts.p[1] = w4_part(qw_up, scales_up, zeros_up, zero_bias_up, N, act);
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    if (w4a16_rows_pays(M, K, nslab, 2) && w4a16_rows_ok(x, M, K, parts))
+        return launch_w4a16_rows_silu(x, M, K, parts, act, st);
     const GemvCfg cfg = choose_gemv(K / kGroup, nslab * M);
     using Fn = void (*)(const uint16_t*, const uint4*, const uint16_t*, const uint32_t*, uint32_t, const uint4*,
                         const uint16_t*, const uint32_t*, uint32_t, uint16_t*, int, int, int);

@@ -1,0 +1,48 @@
+// w4a16_rows.h -- launch interfaces shared by the W4A16 entry points that take
+// several activation rows: the few-row kernel (w4a16_rows.hip), and the list of
+// weights that share one x.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+namespace mcv {
+
+// Up to four slab-64 weights read by one launch over the same x.
+constexpr int kMaxParts = 4;
+struct W4Part {
+    const uint4* qw;
+    const uint16_t* scales;
+    const uint32_t* zeros;
+    uint16_t* out;         // fp16 [M][N]
+    int N;
+    int Npad;
+    int end;               // running total of the launch's column units up to and including this part
+    uint32_t zero_bias;
+};
+struct W4Parts {
+    W4Part p[kMaxParts];
+    int count;
+};
+
+// True where the few-row kernels are the faster ones for M rows over `nslab`
+// slabs of `parts` weights.
+bool w4a16_rows_pays(int64_t M, int64_t K, int64_t nslab, int parts);
+
+// True where the few-row kernels can run this call: at least 2 rows, x
+// 16-byte aligned, x and every packed weight below 2 GiB (32-bit buffer
+// offsets).
+bool w4a16_rows_ok(const void* x, int64_t M, int64_t K, const W4Parts& parts);
+
+// out_i = x . W_i for every part (`end` is set here).
+int launch_w4a16_rows(const void* x, int64_t M, int64_t K, W4Parts parts, hipStream_t stream);
+
+// act = silu(x . gate) * (x . up): parts.p[0] is gate, p[1] up, both [K][N];
+// the sums are launch_w4a16_rows' and round to fp16 before silu_mul_f16.
+int launch_w4a16_rows_silu(const void* x, int64_t M, int64_t K, W4Parts parts, void* act, hipStream_t stream);
+
+// The kernel's configuration for M x K over `cols` padded columns, as text.
+const char* w4a16_rows_name(int64_t M, int64_t K, int64_t nslab);
+
+}  // namespace mcv

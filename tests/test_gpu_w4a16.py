@@ -590,3 +590,29 @@ def test_lm_head_slots_on_side_stream(mcv, oracle, cuda):
         assert head.read_slots_token(tag) == want[i % 2]
     bound = head.bind(xs[1], stream=side, route="slots")
     assert head.read_slots_token(bound()) == want[1]
+
+
+# Several rows: the few-row kernels at the edges of their 16-row blocks, of the
+# trips over K (28 and 31 groups: the last one partly or wholly out of range)
+# and of the wide kernel's column units; the row counts on both sides of the
+# GEMM's start; ragged N and the GPTQ zero bias.
+@pytest.mark.parametrize("M,K,N,zb", [(2, 3584, 8, 1), (5, 1024, 3584, 0), (16, 3968, 136, 1), (17, 128, 1000, 0),
+                                      (32, 3584, 520, 1), (33, 2048, 520, 0), (48, 2176, 1000, 1), (7, 1024, 51272, 0),
+                                      (18, 640, 25672, 1), (64, 1024, 25608, 0), (40, 256, 98312, 1)],
+                         ids=lambda v: str(v))
+def test_several_rows_vs_oracle(mcv, oracle, cuda, M, K, N, zb):
+    x, qweight, qzeros, scales, _ = _case(4000 + M + K + N, M, K, N)
+    w = _dev_weight(mcv, qweight, qzeros, scales)
+    if zb:
+        w = mcv.W4A16QuantizedWeight(w.qweight, w.scales, w.zeros, K, N, 1)
+    q8 = oracle.unpack_awq(qweight, qzeros) - np.int8(zb)
+    got = _host_f32(mcv.matmul_w4a16(_to_dev(x), w))
+    xf = x.view(np.float16).astype(np.float64)
+    wf = q8.astype(np.float64) * np.repeat(scales.view(np.float16).astype(np.float64), 128, axis=0)
+    ref = xf @ wf
+    # one rounding of the output and fp32 sums of K products; the GEMM's 64 x 64
+    # and 128-row tiles round each weight to fp16 first
+    rounded = "<64, 2" in mcv.lib().mcv_w4a16_gemm_kernel_name(M, K, N, 1).decode()
+    mag = np.abs(xf) @ np.abs(wf)
+    bound = 2.0 ** -11 * np.abs(ref) + (K * 2.0 ** -24 + (2.0 ** -11 if rounded else 0)) * mag + 2.0 ** -24
+    assert (np.abs(got - ref) <= bound).all(), float((np.abs(got - ref) - bound).max())
