@@ -219,7 +219,8 @@ int mcv_w4a16_gemm_sk(const void* x_dev, int64_t M, int64_t K, int64_t N,
                       int groups_per_stage, int k_parts, int weights_in_registers, int tile_order,
                       int splits, void* workspace_dev, int64_t workspace_bytes, mcv_stream_t stream);
 
-/* The two kernels behind mcv_w4a16_gemm, callable directly (same contract). */
+/* The two sides of mcv_w4a16_gemm, callable directly (same contract): the GEMV
+ * and few-row kernels, and the MFMA GEMM. */
 int mcv_w4a16_gemv(const void* x_dev, int64_t M, int64_t K, int64_t N,
                    const void* qw_dev, const void* scales_dev, const void* zeros_dev,
                    int zero_bias, void* out_dev, mcv_stream_t stream);
@@ -228,11 +229,12 @@ int mcv_w4a16_gemm_mfma(const void* x_dev, int64_t M, int64_t K, int64_t N,
                         int zero_bias, void* out_dev, mcv_stream_t stream);
 
 /* Decode MLP front half in one launch: act[M][N] = silu(x . Wgate) * (x . Wup)
- * with gate and up rounded to fp16 first, exactly as two mcv_w4a16_gemv calls
- * followed by mcv_silu_mul produce it (bit-identical).  Both weights are K x N
+ * with gate and up rounded to fp16 first, as two mcv_w4a16_gemv calls followed
+ * by mcv_silu_mul produce it (bit-identical up to 32 rows; beyond, the same
+ * exact q - z and fp32 sums in the GEMM's order).  Both weights are K x N
  * slab-64.  Replaces the gate matmul + up matmul + silu_mul sequence of the
  * decoder layers' MLP (src/csrc/lib/decoder_layer.cpp:1029-1046, silu_mul
- * src/csrc/lib/ops.cpp:437-456).  Meant for decode-sized M (GEMV kernel). */
+ * src/csrc/lib/ops.cpp:437-456).  Any M. */
 int mcv_w4a16_gate_up_silu(const void* x_dev, int64_t M, int64_t K, int64_t N,
                            const void* qw_gate_dev, const void* scales_gate_dev, const void* zeros_gate_dev,
                            int zero_bias_gate, const void* qw_up_dev, const void* scales_up_dev,
@@ -295,8 +297,9 @@ typedef struct mcv_w4a16_part {
 /* Up to four projections of the same x [M][K] in one launch: the decode
  * step's q/k/v (src/csrc/lib/decoder_layer.cpp:970-972) or qkv and z
  * (:1108-1110), which the reference dispatches one matmul_decode_dispatch at a
- * time.  Each part's output equals mcv_w4a16_gemv on that weight when both
- * split K the same way (every K = 1024 decode shape). */
+ * time.  Each part's output equals mcv_w4a16_gemv on that weight when both run
+ * the same kernel and split K the same way (M = 1: every K = 1024 decode shape);
+ * at larger M the fp32 sums may be added in another order.  Any M. */
 int mcv_w4a16_gemv_multi(const void* x_dev, int64_t M, int64_t K, const mcv_w4a16_part* parts, int n_parts,
                          mcv_stream_t stream);
 

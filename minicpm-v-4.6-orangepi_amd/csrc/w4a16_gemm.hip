@@ -15,7 +15,6 @@
 
 #include "common.h"
 #include "w4a16_gemm_sk.h"
-#include "w4a16_rows.h"
 
 namespace mcv {
 
@@ -23,12 +22,13 @@ int launch_w4a16_gemv(const void* x, int64_t M, int64_t K, int64_t N, const void
                       const void* zeros, int zero_bias, void* out, hipStream_t stream);
 int gemv_ksplit(int64_t G, int64_t blocks);
 
-// The few-row kernels aside (w4a16_rows_pays comes first): the GEMV streams the weights once per row and still beats the
-// MFMA GEMM, whose tile count is M/TM * N/TN, until the output reaches about
-// 64K elements (MI355X, rotated weights: K=1024 N=3584 M=16 5.7 us against
-// 7.0; K=3584 N=1024 M=48 12.4 against 12.5; K=1024 N=6144 crosses over near
-// M=11).
-bool w4a16_prefers_gemv(int64_t M, int64_t N) { return M >= 1 && (M < 8 || M * N < 65536); }
+// The few-row kernels aside (w4a16_rows_pays comes first): the GEMV streams the
+// weights once per row and still beats the MFMA GEMM, whose tile count is M/TM
+// * N/TN, until the output reaches about 64K elements; with more than 32 rows
+// only on a short K or a grid of one workgroup per CU (MI355X, rotated weights:
+// M=48 N=1024 K=1024 4.67 us against 4.85; M=40 N=1024 K=3584 12.9 against 7.2,
+// K=2048 8.4 against 6.5).
+bool small_output(int64_t M, int64_t N) { return M >= 1 && (M < 8 || M * N < 65536); }
 
 // The GEMM's configuration for M x K x N.  First the largest tile whose grid
 // gives 200-256 workgroups, one tile each (a workgroup per CU): 128 x 256
@@ -97,18 +97,23 @@ SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split) {
     return finish(c);
 }
 
+bool w4a16_prefers_gemv(int64_t M, int64_t K, int64_t N) {
+    return small_output(M, N) && (M <= 32 || K <= 1024 || M * ceil_div(N, kSlab) <= 256);
+}
+
 namespace {
 
 // The GEMV or (through launch_w4a16_gemv) the few-row kernels take this call.
-// The few-row kernels need an aligned x and 32-bit offsets; a call without them
-// goes where it always went.
+// The few-row kernels and the GEMM need an aligned x and 32-bit offsets; a small
+// output without them runs the GEMV, which needs neither.
 bool takes_gemv(const void* x, int64_t M, int64_t K, int64_t N) {
-    if (w4a16_prefers_gemv(M, N)) return true;
-    if (x == nullptr || M < 2 || K <= 0 || K % kGroup != 0 || N <= 0 || N > (int64_t(1) << 30)) return false;
+    if (w4a16_prefers_gemv(M, K, N)) return true;
+    if (x == nullptr || M < 2 || K <= 0 || K % kGroup != 0 || N <= 0 || N > (int64_t(1) << 30)) return small_output(M, N);
     W4Parts parts{};
     parts.count = 1;
     parts.p[0].Npad = static_cast<int>(ceil_div(N, kSlab) * kSlab);
-    return w4a16_rows_pays(M, K, ceil_div(N, kSlab), 1) && w4a16_rows_ok(x, M, K, parts);
+    if (w4a16_rows_pays(M, K, ceil_div(N, kSlab), 1) && w4a16_rows_ok(x, M, K, parts)) return true;
+    return small_output(M, N) && (reinterpret_cast<uintptr_t>(x) % 16 != 0 || !w4a16_sk_fits(M, K, parts));
 }
 
 int check_gemm_args(const void* x, int64_t M, int64_t K, int64_t N, const void* qw, const void* scales,
@@ -153,7 +158,7 @@ int mcv_w4a16_gemm_mfma(const void* x, int64_t M, int64_t K, int64_t N, const vo
 }
 
 int64_t mcv_w4a16_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N) {
-    if (M < 1 || K <= 0 || N <= 0 || K % kGroup != 0 || w4a16_prefers_gemv(M, N) ||
+    if (M < 1 || K <= 0 || N <= 0 || K % kGroup != 0 || w4a16_prefers_gemv(M, K, N) ||
         w4a16_rows_pays(M, K, ceil_div(N, kSlab), 1))
         return 0;
     return w4a16_sk_workspace_bytes(M, N, choose_gemm(M, K, N, true));
@@ -186,7 +191,7 @@ const char* mcv_w4a16_gemm_kernel_name(int64_t M, int64_t K, int64_t N, int with
         g_kernel_name = "none (bad shape)";
     } else if (w4a16_rows_pays(M, K, ceil_div(N, kSlab), 1)) {
         g_kernel_name = w4a16_rows_name(M, K, ceil_div(N, kSlab));
-    } else if (w4a16_prefers_gemv(M, N)) {
+    } else if (w4a16_prefers_gemv(M, K, N)) {
         std::snprintf(buf, sizeof(buf), "w4a16_gemv_kernel<%d, 1, 0> (grid %lld x %lld)",
                       gemv_ksplit(K / kGroup, ceil_div(N, kSlab) * M), (long long)ceil_div(N, kSlab), (long long)M);
         g_kernel_name = buf;

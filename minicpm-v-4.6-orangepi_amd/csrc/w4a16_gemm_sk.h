@@ -6,6 +6,8 @@
 
 #include <cstdint>
 
+#include "w4a16_rows.h"
+
 namespace mcv {
 
 // Tile TM rows x 32 * nwv columns (nwv half-slabs of 32 columns), ns stages
@@ -39,5 +41,15 @@ bool w4a16_sk_config_valid(int64_t M, int64_t K, int64_t N, const SkConfig& c);
 int launch_w4a16_gemm_sk(const void* x, int64_t M, int64_t K, int64_t N, const void* qw, const void* scales,
                          const void* zeros, int zero_bias, void* out, const SkConfig& c, void* ws, int64_t ws_bytes,
                          hipStream_t stream);
+
+// Several weights over one x (no K split): out_i = x . W_i per part, or with
+// `act` part 0 the gate and part 1 the up weight of silu(x . gate) * (x . up).
+int launch_w4a16_gemm_sk_parts(const void* x, int64_t M, int64_t K, const W4Parts& parts, void* act, const SkConfig& c,
+                               hipStream_t stream);
+// True where the GEMM's 32-bit buffer offsets cover this call.
+bool w4a16_sk_fits(int64_t M, int64_t K, const W4Parts& parts);
+// The configuration the dispatch (w4a16_gemm.hip) takes for M x K x N.
+SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split);
+bool w4a16_prefers_gemv(int64_t M, int64_t K, int64_t N);
 
 }  // namespace mcv

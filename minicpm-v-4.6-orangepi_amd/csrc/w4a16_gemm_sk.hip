@@ -37,10 +37,14 @@
 // the two 4-byte words of its k-octet parity (l/32) -- a pair of chunks in one
 // ds_read_b128 (the half-waves read one chunk each) and two v_permlane32_swap
 // (a lane-per-word read, 16 bytes apart, costs ~12 bank-conflict cycles) --
-// eight words per group, one per k16 step, each widened into the 8-value
-// fp16 operand RNE((q - z) * s) -- the values mcv_w4a16_dequant materialises
-// ((1024 + q) - (1024 + z) exact through the fp16 exponent, times s, one
-// rounding).
+// eight words per group, one per k16 step, each widened into the exact 8-value
+// fp16 operand q - z (widen_exact).
+// EX = 1: those operands feed the MFMAs, each group's fp32 sum then meets its
+// scale in one fma per result (the GEMV's arithmetic; a lane's 16 results of a
+// block are 16 consecutive columns, so their scales are 32 contiguous bytes).
+// EX = 0: the operand is multiplied by s first, fp16 RNE((q - z) * s), the
+// values mcv_w4a16_dequant materialises.  EX trades 4 packed multiplies per k16
+// step for 16 TM/32 fmas per group and 16 TM/32 registers (one_exact).
 //
 // WR = 1: the packed chunks, zero words and scales skip LDS.  A wave's
 // weight columns are its own (no other wave of the tile reads them), so each
@@ -71,6 +75,12 @@
 //
 // Output: fp16 through LDS, whole tile rows per store instruction,
 // non-temporal (full lines go straight to HBM while other tiles compute).
+//
+// Several weights over one x (kParts: q/k/v or qkv and z; kSilu: gate and up with
+// the activation) run as one grid over their column tiles, always EX: a GEMV
+// row per activation row, which these calls ran before, is exact too.  MI355X,
+// us before / after, K=1024: qkv + z (8192 columns) M=77 37 / 6.8, M=1100 430 /
+// 31.5; gate + up (2 x 3584) M=77 34 / 6.7, M=1100 385 / 20.9.
 //
 // The reference has no M > 1 quantised path: its prefill runs dense fp16
 // aclnnMm through matmul_b_transposed (src/csrc/lib/decoder_layer.cpp:459-462,
@@ -110,7 +120,9 @@ __device__ __forceinline__ int xcd_run(int b, int total) {
     return x * per + (x < rem ? x : rem) + i;
 }
 
-template <int TM, int NWV, int NS, int KG, int KW, int WR>
+constexpr int kOne = 0, kParts = 1, kSilu = 2;
+
+template <int TM, int NWV, int NS, int KG, int KW, int WR, int EX>
 struct CfgS {
     static constexpr int WS = NWV / 2;                   // slabs per tile
     static constexpr int TN = 32 * NWV;                  // columns per tile
@@ -128,8 +140,8 @@ struct CfgS {
     static constexpr int PB = WR ? 0 : (4 * KG * WS) / NWT;   // packed chunks, 1 KiB each
     static constexpr int PZ = WR ? 0 : (2 * KG * WS) / NWT;   // zero words or scales of one (group, slab)
     // WR: each wave loads its own part of the stage's weights into registers
-    // instead (per group: two chunk pairs, the zero word, the scale)
-    static constexpr int PR = WR ? 4 * GW : 0;
+    // instead (per group: two chunk pairs, the zero word, the scales)
+    static constexpr int PR = WR ? (EX ? 5 : 4) * GW : 0;
     static constexpr int P = PA + PB + PZ + PR;
     // after the K loop each wave owns OB of the tile's MB row blocks of its
     // half-slab (k-part kp owns blocks kp * OB ..), the KW partial sums added
@@ -154,12 +166,20 @@ struct CfgS {
     static_assert(KW == 1 || NWV * MB * 16 * 64 * 4 <= STAGE, "k-part exchange space");
 };
 
-template <int TM, int NWV, int NS, int KG, int KW, int WR>
+// kOne: out = x . W (part 0).  kParts: out_i = x . W_i for every part, the
+// column tiles running over the parts one after another (`end` counts tiles;
+// picking the part costs ~0.15 us at the start).  kSilu: act = silu(x .
+// gate) * (x . up), part 0 the gate and part 1 the up weight: the first half of
+// a tile's half-slabs are gate columns, the second half the up columns of the
+// same output columns, and the epilogue combines the two halves of the staged
+// fp16 tile -- the roundings of two launches and silu_mul.
+template <int TM, int NWV, int NS, int KG, int KW, int WR, int KIND, int EX>
 __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
-    const uint16_t* __restrict__ x, const uint4* __restrict__ qw, const uint16_t* __restrict__ scales,
-    const uint32_t* __restrict__ zeros, uint32_t zero_bias, uint16_t* __restrict__ out, int M, int K, int N,
-    int nslab, int m_tiles, int n_tiles, int S, int order, uint8_t* __restrict__ ws, uint32_t ws_bytes) {
-    using C = CfgS<TM, NWV, NS, KG, KW, WR>;
+    const uint16_t* __restrict__ x, W4Parts parts, uint16_t* __restrict__ act, int M, int K, int m_tiles, int n_tiles,
+    int S, int order, uint8_t* __restrict__ ws, uint32_t ws_bytes) {
+    using C = CfgS<TM, NWV, NS, KG, KW, WR, EX>;
+    constexpr bool SILU = KIND == kSilu;
+    constexpr int HO = SILU ? NWV / 2 : NWV;             // output half-slabs per tile
     __shared__ __attribute__((aligned(1024))) uint8_t lds0[C::STAGE];
     __shared__ __attribute__((aligned(1024))) uint8_t lds1[C::STAGE];
     __shared__ __attribute__((aligned(1024))) uint8_t lds2[NS > 2 ? C::STAGE : 16];
@@ -196,7 +216,21 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
         tn = tile - tm * n_tiles;
     }
     const int m0 = tm * TM;
-    const int Npad = nslab * kSlab;
+    // the part this tile's columns belong to (constant indices only: the
+    // kernel arguments stay in SGPRs)
+    W4Part P = parts.p[0];
+    if constexpr (KIND == kParts) {
+        int first = 0;
+#pragma unroll
+        for (int i = 1; i < kMaxParts; ++i)
+            if (i < parts.count && tn >= parts.p[i - 1].end) {
+                P = parts.p[i];
+                first = parts.p[i - 1].end;
+            }
+        tn -= first;
+    }
+    const int N = P.N, Npad = P.Npad, nslab = Npad / kSlab;
+    uint16_t* __restrict__ const out = SILU ? act : P.out;
     const int CK = K / kChunkK;
     const int G = K / kGroup;
     // split p takes stages [p U / S, (p+1) U / S) of the U = G / KG stages
@@ -209,9 +243,14 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
     const int rows_here = M - m0 < TM ? M - m0 : TM;
     const __amdgpu_buffer_rsrc_t xr =
         rsrc_s(x + static_cast<size_t>(m0) * K, static_cast<uint32_t>(rows_here) * K * 2u);
-    const __amdgpu_buffer_rsrc_t qr = rsrc_s(qw, static_cast<uint32_t>(nslab) * CK * kSlab * 16u);
-    const __amdgpu_buffer_rsrc_t sr = rsrc_s(scales, static_cast<uint32_t>(G) * Npad * 2u);
-    const __amdgpu_buffer_rsrc_t zr = rsrc_s(zeros, static_cast<uint32_t>(G) * (Npad >> 3) * 4u);
+    // the weight a slab of the tile belongs to: in the SILU tile slabs (with WR,
+    // half-slabs) from the middle on are the up weight's
+    auto q_of = [&](bool up) { return rsrc_s(SILU && up ? parts.p[1].qw : P.qw, static_cast<uint32_t>(nslab) * CK * kSlab * 16u); };
+    auto s_of = [&](bool up) { return rsrc_s(SILU && up ? parts.p[1].scales : P.scales, static_cast<uint32_t>(G) * Npad * 2u); };
+    auto z_of = [&](bool up) { return rsrc_s(SILU && up ? parts.p[1].zeros : P.zeros, static_cast<uint32_t>(G) * (Npad >> 3) * 4u); };
+    constexpr int SO = SILU && !WR ? C::WS / 2 : C::WS;  // output slabs per tile of the LDS path
+    const bool hup = SILU && hw >= HO;                   // this wave's half-slab is the up weight's
+    const uint32_t zero_bias = hup ? parts.p[1].zero_bias : P.zero_bias;
 
     // This wave's copies of a stage, each lane's offset fixed here; the
     // stage's advance rides in the scalar offset.  The buffer range check
@@ -233,7 +272,8 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
     // chunk t % (4 KG) of that slab's stage (group c / 4, 32-k chunk c % 4)
     const int bitem = wave * C::PB;
     const int bslab_t = bitem / (4 * KG);
-    const int bslab = tn * C::WS + bslab_t;
+    const int bslab = tn * SO + bslab_t % SO;
+    const __amdgpu_buffer_rsrc_t bqr = q_of(bslab_t >= SO);
     const bool bslab_live = bslab < nslab;
     const uint32_t qoff = (static_cast<uint32_t>(bslab) * CK * kSlab * 16u + lane * 16u) | (bslab_live ? 0u : 0x80000000u);
     const int bchunk = bitem % (4 * KG);
@@ -241,14 +281,14 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
     // t / (2 KG), then zero words (kind 0) or scales (kind 1), then group
     const int zitem = wave * C::PZ;
     const int zslab_t = zitem / (2 * KG);
-    const int zslab = tn * C::WS + zslab_t;
+    const int zslab = tn * SO + zslab_t % SO;
     const bool zslab_live = zslab < nslab;
     const bool zkind = (zitem % (2 * KG)) / KG == 0;
     const int zgrp = zitem % KG;                         // first group of this wave's items
     const uint32_t zsoff = zkind ? ((static_cast<uint32_t>(zslab) * 32u + lane * 4u) | (lane < 8 && zslab_live ? 0u : 0x80000000u))
                                  : ((static_cast<uint32_t>(zslab) * 128u + lane * 4u) | (lane < 32 && zslab_live ? 0u : 0x80000000u));
     const int zsstride = zkind ? (Npad >> 3) * 4 : Npad * 2;
-    const __amdgpu_buffer_rsrc_t zsr = zkind ? zr : sr;
+    const __amdgpu_buffer_rsrc_t zsr = zkind ? z_of(zslab_t >= SO) : s_of(zslab_t >= SO);
     const int zsdst = C::Z_OFF + zslab_t * 512 + (zkind ? 0 : 256);   // + group * WS * 512
 
     // WR: this wave's weights of stage kt land in register slot kt % NS (the
@@ -257,14 +297,23 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
     // its column -- the lower half-wave fetches the first chunk of a pair,
     // the upper half the second, as the LDS path's ds_read_b128 does -- plus
     // the column's zero word and scale.  Padding slabs get bit 31 (read zero).
-    const int col = 32 * (hw & 1) + (lane & 31);         // this lane's column inside its slab
-    const int wslab = tn * C::WS + (hw >> 1);
+    const int hs = tn * HO + hw % HO;                    // this wave's half-slab of its weight
+    // This lane's column inside its slab, as operand row i = l%32 of the MFMA:
+    // i = 8 g + 4 b + e takes column 16 b + 4 g + e of the half-slab, so the
+    // result's register r (operand row 8 (r/4) + 4 (l/32) + r%4) is column
+    // 16 (l/32) + r: 16 consecutive columns per lane.
+    const int col = 32 * (hs & 1) + 16 * ((lane >> 2) & 1) + 4 * ((lane >> 3) & 3) + (lane & 3);
+    const int wslab = hs >> 1;
+    const __amdgpu_buffer_rsrc_t qr = q_of(hup), sr = s_of(hup), zr = z_of(hup);
     const uint32_t wdead = wslab < nslab ? 0u : 0x80000000u;
     const uint32_t wq_off = (static_cast<uint32_t>(wslab) * CK * kSlab * 16u + h * 1024u + col * 16u) | wdead;
     const uint32_t wz_off = (static_cast<uint32_t>(wslab) * 32u + (col >> 3) * 4u) | wdead;
-    const uint32_t ws_off = (static_cast<uint32_t>(wslab) * 128u + col * 2u) | wdead;
+    const int scol = EX ? 32 * (hs & 1) + 16 * h : col;  // first column whose scale this lane needs
+    const uint32_t ws_off = (static_cast<uint32_t>(wslab) * 128u + scol * 2u) | wdead;
     uint4 rq[WR ? NS : 1][2 * C::GW];
-    uint32_t rz[WR ? NS : 1][C::GW], rs[WR ? NS : 1][C::GW];
+    uint32_t rz[WR ? NS : 1][C::GW];
+    uint32_t rs[WR && !EX ? NS : 1][C::GW];              // scale of the lane's operand column
+    half8_t rs16[WR && EX ? NS : 1][C::GW][2];           // EX: scales of its 16 result columns
 
     auto issue_item = [&](int kt, uint8_t* dst, int it, int slot) {
         const int kc = kt < KT ? kt : KT - 1;
@@ -272,18 +321,21 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
         if (it < C::PA) {
             dma16_s(xr, dst + (wave * C::PA + it) * kLine, xoff[it], g * 256);
         } else if (WR) {
-            const int r = it - C::PA, j = r / 4, kind = r % 4;
+            const int r = it - C::PA, j = r / (4 + EX), kind = r % (4 + EX);
             const int grp = g + kp * C::GW + j;
             if (kind < 2)
                 rq[slot][2 * j + kind] = __builtin_bit_cast(
                     uint4, __builtin_amdgcn_raw_buffer_load_b128(qr, wq_off, (grp * 4 + 2 * kind) * kSlab * 16, 0));
             else if (kind == 2)
                 rz[slot][j] = __builtin_amdgcn_raw_buffer_load_b32(zr, wz_off, grp * (Npad >> 3) * 4, 0);
+            else if constexpr (EX)
+                rs16[slot][j][kind - 3] = __builtin_bit_cast(
+                    half8_t, __builtin_amdgcn_raw_buffer_load_b128(sr, ws_off + 16u * (kind - 3), grp * Npad * 2, 0));
             else
                 rs[slot][j] = __builtin_amdgcn_raw_buffer_load_b16(sr, ws_off, grp * Npad * 2, 0);
         } else if (it < C::PA + C::PB) {
             const int c = bchunk + (it - C::PA);
-            dma16_s(qr, dst + C::A_BYTES + (bslab_t * 4 * KG + c) * kLine, qoff, (g * 4 + c) * kSlab * 16);
+            dma16_s(bqr, dst + C::A_BYTES + (bslab_t * 4 * KG + c) * kLine, qoff, (g * 4 + c) * kSlab * 16);
         } else {
             const int j = zgrp + (it - C::PA - C::PB);   // group j of the stage
             dma4_s(zsr, dst + zsdst + j * C::WS * 512, zsoff, (g + j) * zsstride);
@@ -297,9 +349,12 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
     uint32_t vmagic;
     asm("v_mov_b32 %0, 0x64006400" : "=v"(vmagic));
     const uint32_t mlo = __builtin_amdgcn_readfirstlane(0x000F000Fu);
+    const uint32_t mhi = __builtin_amdgcn_readfirstlane(0x00F000F0u);
+    const half2_t sixteenth = as_h2(0x2C002C00u);        // half2(1/16)
     const uint32_t zsh = (col & 7) * 4;
 
-    float16_t acc[C::MB];
+    // acc: the sums so far; EX: gacc the current group's sum of x (q - z)
+    float16_t acc[C::MB], gacc[EX ? C::MB : 1];
 #pragma unroll
     for (int i = 0; i < C::MB; ++i)
 #pragma unroll
@@ -316,29 +371,22 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
     // this wave's chunks start at group kp GW of its slab's stage
     const int b_off = C::A_BYTES + ((hw >> 1) * 4 * KG + 4 * kp * C::GW + h) * kLine + col * 16;
     const int z_off = C::Z_OFF + kp * C::GW * C::WS * 512 + (hw >> 1) * 512 + (col >> 3) * 4;
-    const int s_off = C::Z_OFF + kp * C::GW * C::WS * 512 + (hw >> 1) * 512 + 256 + col * 2;
+    const int s_off = C::Z_OFF + kp * C::GW * C::WS * 512 + (hw >> 1) * 512 + 256 + scol * 2;
 
     uint32_t q[C::STEPS];                                // the wave's words of a stage, one per k16 step
-    uint32_t zza[C::GW], ssa[C::GW];                     // per group of the wave's part of a stage
-#pragma unroll
-    for (int j = 0; j < C::GW; ++j) zza[j] = ssa[j] = 0;
+    half2_t zlo[C::GW], zhi[C::GW];                      // per group: half2(1024 + z), half2(-(64 + z))
+    half2_t ss[EX ? 1 : C::GW];                          // half2(scale) of the operand column
+    half8_t sc[EX ? C::GW : 1][2];                       // EX, LDS path: the stage's scales
     half8_t af[2][C::MB], bf[2];
     auto widen = [&](int s, half8_t& b) {
-        const uint32_t w = q[s];
-        const uint32_t zz = zza[s / 8], ss = ssa[s / 8];
-        uint32_t t[4];
+        b = widen_exact(q[s], zlo[s / 8], zhi[s / 8], mlo, mhi, vmagic, sixteenth);
+        if constexpr (!EX)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) t[j] = and_or_b32(j ? w >> (4 * j) : w, mlo, vmagic);
-        half2_t d[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) d[j] = as_h2(t[j]) - as_h2(zz);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) d[j] = d[j] * as_h2(ss);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            b[2 * j] = d[j][0];
-            b[2 * j + 1] = d[j][1];
-        }
+            for (int e = 0; e < 4; ++e) {
+                const half2_t v = half2_t{b[2 * e], b[2 * e + 1]} * ss[s / 8];
+                b[2 * e] = v[0];
+                b[2 * e + 1] = v[1];
+            }
     };
     auto read_a = [&](const uint8_t* src, int s, half8_t* dst) {
 #pragma unroll
@@ -359,25 +407,51 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
             q[2 * c + 1] = s2[0];                        // word 2 + h of chunk c
             q[2 * c + 3] = s2[1];                        // word 2 + h of chunk c + 1
         }
-        uint32_t zw[C::GW], sh[C::GW];
+        uint32_t zw[C::GW];
 #pragma unroll
-        for (int j = 0; j < C::GW; ++j) {
+        for (int j = 0; j < C::GW; ++j)
             zw[j] = WR ? rz[slot][j] : *reinterpret_cast<const uint32_t*>(src + z_off + j * C::WS * 512);
-            sh[j] = WR ? rs[slot][j] & 0xffffu : *reinterpret_cast<const uint16_t*>(src + s_off + j * C::WS * 512);
-        }
         read_a(src, 0, af[0]);
 #pragma unroll
         for (int j = 0; j < C::GW; ++j) {
-            zza[j] = (0x6400u + ((zw[j] >> zsh) & 15u) + zero_bias) * 0x10001u;
-            ssa[j] = sh[j] * 0x10001u;
+            const uint32_t z = ((zw[j] >> zsh) & 15u) + zero_bias;
+            zlo[j] = as_h2((0x6400u + z) * 0x10001u);
+            zhi[j] = as_h2((0xD400u + (z << 4)) * 0x10001u);
+            if constexpr (!EX) {
+                const uint32_t sv = WR ? rs[slot][j] & 0xffffu
+                                       : *reinterpret_cast<const uint16_t*>(src + s_off + j * C::WS * 512);
+                ss[j] = as_h2(sv * 0x10001u);
+            }
         }
     };
-    auto mfmas = [&](int cur, int lo, int hi) {
+    // EX, LDS path: the scales of group j of `src`'s stage, read before the
+    // barrier that frees it
+    auto read_scales = [&](const uint8_t* src, int j) {
+        if constexpr (EX && !WR)
 #pragma unroll
-        for (int i = lo; i < hi; ++i)
-            acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[cur], af[cur][i], acc[i], 0, 0, 0);
+            for (int c = 0; c < 2; ++c)
+                sc[j][c] = *reinterpret_cast<const half8_t*>(src + s_off + j * C::WS * 512 + 16 * c);
     };
-    constexpr int kV = (15 + C::MB - 1) / C::MB;         // widening VALU per MFMA
+    auto mfmas = [&](int cur, int lo, int hi, bool first) {
+#pragma unroll
+        for (int i = lo; i < hi; ++i) {
+            if constexpr (EX)
+                gacc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[cur], af[cur][i], first ? float16_t{} : gacc[i], 0, 0, 0);
+            else
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[cur], af[cur][i], acc[i], 0, 0, 0);
+        }
+    };
+    // EX: group j of the stage is complete, its sums meet their scales
+    auto fold = [&](int j, int slot) {
+        if constexpr (EX)
+#pragma unroll
+            for (int i = 0; i < C::MB; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    acc[i][r] = fmaf(gacc[i][r], static_cast<float>(WR ? rs16[slot][j][r >> 3][r & 7] : sc[j][r >> 3][r & 7]),
+                                     acc[i][r]);
+    };
+    constexpr int kV = ((EX ? 9 : 13) + C::MB - 1) / C::MB;   // widening VALU per MFMA
 
     // One stage from `cur`: steps 0-6 produce step s+1's operands while step
     // s's MFMAs run and spread the copies of stage kt + NS - 1 into `prv`
@@ -393,7 +467,7 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
             for (int it = lo; it < hi; ++it) issue_item(kt + NS - 1, prv, it, (u + NS - 1) % NS);
             read_a(cur, s + 1, af[n]);
             widen(s + 1, bf[n]);
-            mfmas(c, 0, C::MB);
+            mfmas(c, 0, C::MB, s % 8 == 0);
 #pragma unroll
             for (int i = 0; i < C::MB; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                  // DS read
@@ -402,18 +476,21 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
                 __builtin_amdgcn_sched_group_barrier(0x002, kV, 0);                 // VALU
             }
             __builtin_amdgcn_sched_barrier(0);
+            if (s % 8 == 7) fold(s / 8, u);              // (two groups per stage and wave)
+            if (s % 8 == 6) read_scales(cur, s / 8);
         }
         static_assert(C::STEPS % 2 == 0, "the last step uses operand set 1");
-        mfmas(1, 0, (C::MB + 1) / 2);
+        mfmas(1, 0, (C::MB + 1) / 2, false);
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         wait_vmcnt_s<C::P * (NS - 2)>();
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         head(nxt, (u + 1) % NS);
-        mfmas(1, (C::MB + 1) / 2, C::MB);
+        mfmas(1, (C::MB + 1) / 2, C::MB, false);
         __builtin_amdgcn_sched_barrier(0);
         widen(0, bf[0]);
+        fold(C::GW - 1, u);
     };
 
 #pragma unroll
@@ -545,23 +622,16 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
     }
 
     // ---- fp16 epilogue.  Owned block ii (row block ib0 + ii): register r of
-    // lane l holds output row 32 (ib0 + ii) + l%32 and column 8 (r/4) +
-    // 4 (l/32) + r%4 of the half-slab's 32; swapping the upper lanes of quad g
-    // with the lower lanes of quad g+1 leaves lane l with the 8 consecutive
-    // columns 8 g + 8 (l/32), g even.
-    auto pack = [&](int ii, int g, uint32_t (&pk)[4]) {
+    // lane l holds output row 32 (ib0 + ii) + l%32 and column 16 (l/32) + r of
+    // the half-slab's 32; chunk c (0 or 1) is columns 16 (l/32) + 8 c ..
+    auto pack = [&](int ii, int c, uint32_t (&pk)[4]) {
 #pragma unroll
-        for (int d = 0; d < 2; ++d) {
-            const uint32_t x0 = f2h(own[ii][4 * g + 2 * d]) | (uint32_t(f2h(own[ii][4 * g + 2 * d + 1])) << 16);
-            const uint32_t x1 = f2h(own[ii][4 * g + 4 + 2 * d]) | (uint32_t(f2h(own[ii][4 * g + 5 + 2 * d])) << 16);
-            const auto sw = __builtin_amdgcn_permlane32_swap(x0, x1, false, false);
-            pk[d] = sw[0];
-            pk[2 + d] = sw[1];
-        }
+        for (int d = 0; d < 4; ++d)
+            pk[d] = f2h(own[ii][8 * c + 2 * d]) | (uint32_t(f2h(own[ii][8 * c + 2 * d + 1])) << 16);
     };
-    const int n0 = tn * C::TN;
+    const int n0 = tn * 32 * HO;
     const bool vec_ok = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-    if (vec_ok) {
+    if (SILU || vec_ok) {
         // the whole tile through LDS (the stage buffers: every wave is past
         // its last operand read after this barrier), then whole rows per
         // store instruction, non-temporal
@@ -574,23 +644,40 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
 #pragma unroll
         for (int ii = 0; ii < C::OB; ++ii)
 #pragma unroll
-            for (int g = 0; g < 4; g += 2) {
+            for (int c = 0; c < 2; ++c) {
                 if (!owns) continue;
                 uint32_t pk[4];
-                pack(ii, g, pk);
-                *reinterpret_cast<uint4*>(srow(32 * (ib0 + ii) + (lane & 31)) + (32 * hw + 8 * g + 8 * h) * 2) =
+                pack(ii, c, pk);
+                *reinterpret_cast<uint4*>(srow(32 * (ib0 + ii) + (lane & 31)) + (32 * hw + 16 * h + 8 * c) * 2) =
                     make_uint4(pk[0], pk[1], pk[2], pk[3]);
             }
         __syncthreads();
-        constexpr int CPR = C::TN / 8;                   // 16-byte chunks per row
+        constexpr int CPR = 4 * HO;                      // 16-byte chunks per output row
         constexpr int RPI = 64 * C::NWT / CPR;           // rows per workgroup-wide pass
-        static_assert(TM % RPI == 0, "row passes");
+        static_assert(TM % RPI == 0 || RPI > TM, "row passes");
         const int cl = static_cast<int>(threadIdx.x) % CPR, rl = static_cast<int>(threadIdx.x) / CPR;
+        if (RPI > TM && rl >= TM) return;
 #pragma unroll
-        for (int it = 0; it < TM / RPI; ++it) {
+        for (int it = 0; it < (RPI > TM ? 1 : TM / RPI); ++it) {
             const int r = it * RPI + rl;
             const int row = m0 + r, c0 = n0 + 8 * cl;
-            const uint4 v = *reinterpret_cast<const uint4*>(srow(r) + cl * 16);
+            uint4 v = *reinterpret_cast<const uint4*>(srow(r) + cl * 16);
+            if constexpr (SILU) {
+                const uint4 u = *reinterpret_cast<const uint4*>(srow(r) + 64 * HO + cl * 16);
+                auto two = [](uint32_t g, uint32_t w) {
+                    return uint32_t(silu_mul_f16(static_cast<uint16_t>(g), static_cast<uint16_t>(w))) |
+                           (uint32_t(silu_mul_f16(static_cast<uint16_t>(g >> 16), static_cast<uint16_t>(w >> 16))) << 16);
+                };
+                v = make_uint4(two(v.x, u.x), two(v.y, u.y), two(v.z, u.z), two(v.w, u.w));
+                if (!vec_ok) {
+                    const uint32_t a[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (row < M && c0 + e < N)
+                            out[static_cast<size_t>(row) * N + c0 + e] = static_cast<uint16_t>(a[e >> 1] >> (16 * (e & 1)));
+                    continue;
+                }
+            }
             if (row < M && c0 < N)
                 __builtin_nontemporal_store(int4_t{static_cast<int>(v.x), static_cast<int>(v.y), static_cast<int>(v.z),
                                                    static_cast<int>(v.w)},
@@ -604,10 +691,10 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
         if (!owns) break;
         const int row = m0 + 32 * (ib0 + ii) + (lane & 31);
 #pragma unroll
-        for (int g = 0; g < 4; g += 2) {
+        for (int c = 0; c < 2; ++c) {
             uint32_t pk[4];
-            pack(ii, g, pk);
-            const int c0 = n0 + 32 * hw + 8 * g + 8 * h;
+            pack(ii, c, pk);
+            const int c0 = n0 + 32 * hw + 16 * h + 8 * c;
             if (row >= M || c0 >= N) continue;
             uint16_t* dst = out + static_cast<size_t>(row) * N + c0;
 #pragma unroll
@@ -617,8 +704,7 @@ __global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
     }
 }
 
-using SkFn = void (*)(const uint16_t*, const uint4*, const uint16_t*, const uint32_t*, uint32_t, uint16_t*, int, int,
-                      int, int, int, int, int, int, uint8_t*, uint32_t);
+using SkFn = void (*)(const uint16_t*, W4Parts, uint16_t*, int, int, int, int, int, int, uint8_t*, uint32_t);
 
 #define MCV_SK_SHAPES(X)                                                                                   \
     X(128, 8, 3, 1, 1, 0) X(128, 4, 3, 1, 1, 0) X(64, 8, 3, 1, 1, 0) X(64, 4, 3, 1, 1, 0) X(32, 4, 3, 1, 1, 0)   \
@@ -626,11 +712,30 @@ using SkFn = void (*)(const uint16_t*, const uint4*, const uint16_t*, const uint
     X(64, 4, 3, 1, 1, 1) X(64, 4, 3, 2, 2, 1) X(64, 4, 4, 2, 2, 1) X(32, 4, 3, 1, 1, 1) X(32, 4, 3, 2, 1, 1)   \
     X(32, 4, 3, 2, 2, 1) X(32, 2, 3, 1, 1, 1) X(32, 2, 3, 2, 2, 1) X(64, 2, 3, 2, 2, 1) X(32, 2, 4, 2, 2, 1)   \
     X(128, 2, 3, 1, 1, 1) X(128, 2, 2, 2, 2, 1) X(64, 2, 3, 1, 1, 1)
+// EX for one weight: where it is at least as fast.  MI355X, us, EX / rounded
+// weights: 32 x 64 M=128 K=3584 7.81 / 8.01, 32 x 128 M=1100 K=3584 19.7 / 21.0,
+// 64 x 128 M=1100 N=3584 16.07 / 16.35; but 128 x 256 (twice the accumulators)
+// M=2048 19.95 / 19.03, and 64 x 64 M=256 7.03 / 6.81.
+constexpr int one_exact(int tm, int nwv, int, int, int, int) { return tm == 32 || (tm == 64 && nwv == 4) ? 1 : 0; }
 
-SkFn pick_sk(int tm, int nwv, int ns, int kg, int kw, int wr) {
-#define MCV_SK_PICK(a, b, c, d, e, f) \
-    if (tm == a && nwv == b && ns == c && kg == d && kw == e && wr == f) return w4a16_gemm_sk_kernel<a, b, c, d, e, f>;
+// what the dispatch picks (choose_gemm), for several weights
+#define MCV_SK_PARTS_SHAPES(X)                                                                             \
+    X(128, 8, 3, 1, 1, 0) X(64, 4, 3, 1, 1, 1) X(64, 4, 3, 2, 2, 1) X(32, 4, 3, 1, 1, 1) X(32, 4, 3, 2, 2, 1)   \
+    X(32, 2, 3, 1, 1, 1) X(32, 2, 3, 2, 2, 1) X(64, 2, 3, 2, 2, 1) X(64, 2, 3, 1, 1, 1)
+
+SkFn pick_sk(int tm, int nwv, int ns, int kg, int kw, int wr, int kind) {
+    const int want[6] = {tm, nwv, ns, kg, kw, wr};
+    auto is = [&](int a, int b, int c, int d, int e, int f) {
+        return want[0] == a && want[1] == b && want[2] == c && want[3] == d && want[4] == e && want[5] == f;
+    };
+#define MCV_SK_PICK(...) \
+    if (kind == kOne && is(__VA_ARGS__)) return w4a16_gemm_sk_kernel<__VA_ARGS__, kOne, one_exact(__VA_ARGS__)>;
     MCV_SK_SHAPES(MCV_SK_PICK)
+#undef MCV_SK_PICK
+#define MCV_SK_PICK(...)                                                              \
+    if (kind == kParts && is(__VA_ARGS__)) return w4a16_gemm_sk_kernel<__VA_ARGS__, kParts, 1>; \
+    if (kind == kSilu && is(__VA_ARGS__)) return w4a16_gemm_sk_kernel<__VA_ARGS__, kSilu, 1>;
+    MCV_SK_PARTS_SHAPES(MCV_SK_PICK)
 #undef MCV_SK_PICK
     return nullptr;
 }
@@ -648,23 +753,44 @@ int64_t w4a16_sk_workspace_bytes(int64_t M, int64_t N, const SkConfig& c) {
 }
 
 bool w4a16_sk_config_valid(int64_t M, int64_t K, int64_t N, const SkConfig& c) {
-    return pick_sk(c.tm, c.nwv, c.ns, c.kg, c.kw, c.wr) != nullptr && c.splits >= 1 && c.splits <= 64 && K % kGroup == 0 &&
+    return pick_sk(c.tm, c.nwv, c.ns, c.kg, c.kw, c.wr, kOne) != nullptr && c.splits >= 1 && c.splits <= 64 && K % kGroup == 0 &&
            (K / kGroup) % c.kg == 0 && c.splits <= K / kGroup / c.kg &&
            (c.splits == 1 || w4a16_sk_tiles(M, N, c) <= kSkMaxSplitTiles);
 }
 
-int launch_w4a16_gemm_sk(const void* x, int64_t M, int64_t K, int64_t N, const void* qw, const void* scales,
-                         const void* zeros, int zero_bias, void* out, const SkConfig& c, void* ws, int64_t ws_bytes,
-                         hipStream_t stream) {
-    SkFn fn = pick_sk(c.tm, c.nwv, c.ns, c.kg, c.kw, c.wr);
-    if (fn == nullptr || !w4a16_sk_config_valid(M, K, N, c))
+bool w4a16_sk_fits(int64_t M, int64_t K, const W4Parts& parts) {
+    if (M < 1 || K > (int64_t(1) << 22) || 128 * K * 2 >= (int64_t(1) << 31)) return false;
+    int64_t cols = 0;
+    for (int i = 0; i < parts.count; ++i) {
+        if (K * parts.p[i].Npad / 2 >= (int64_t(1) << 31)) return false;
+        cols += parts.p[i].Npad;
+    }
+    return ceil_div(M, 32) * ceil_div(cols, 64) <= 0x7fffffff;
+}
+
+namespace {
+
+int launch_sk(const void* x, int64_t M, int64_t K, W4Parts parts, void* act, bool exact, const SkConfig& c, void* ws,
+              int64_t ws_bytes, hipStream_t stream) {
+    const bool silu = act != nullptr;
+    const int64_t N = parts.p[0].N;
+    SkFn fn = pick_sk(c.tm, c.nwv, c.ns, c.kg, c.kw, c.wr, silu ? kSilu : (exact ? kParts : kOne));
+    if (fn == nullptr || !w4a16_sk_config_valid(M, K, N, c) || (c.splits > 1 && (parts.count > 1 || silu)))
         return fail(MCV_ERR_INVALID_ARG,
                     "w4a16 GEMM: no kernel for TM=%d waves=%d NS=%d KG=%d KW=%d WR=%d S=%d at M=%lld K=%lld N=%lld (KG must "
-                    "divide K/128, S be at most K/128/KG, and a split needs at most %d tiles)",
+                    "divide K/128, S be at most K/128/KG, and a split needs one weight and at most %d tiles)",
                     c.tm, c.nwv, c.ns, c.kg, c.kw, c.wr, c.splits, (long long)M, (long long)K, (long long)N,
                     kSkMaxSplitTiles);
-    const int64_t nslab = ceil_div(N, kSlab);
-    const int64_t m_tiles = ceil_div(M, c.tm), n_tiles = ceil_div(nslab, c.nwv / 2);
+    // column tiles over all parts (SILU: gate and up slabs side by side)
+    int64_t nslab = 0, n_tiles = 0, widest = 0;
+    for (int i = 0; i < (silu ? 1 : parts.count); ++i) {
+        const int64_t own = parts.p[i].Npad / kSlab, ns = silu ? 2 * own : own;
+        nslab += ns;
+        widest = own > widest ? own : widest;
+        n_tiles += ceil_div(ns, c.nwv / 2);
+        parts.p[i].end = static_cast<int>(n_tiles);
+    }
+    const int64_t m_tiles = ceil_div(M, c.tm);
     const int64_t total = m_tiles * n_tiles * c.splits;
     const int64_t need = w4a16_sk_workspace_bytes(M, N, c);
     if (c.splits > 1 && (ws == nullptr || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255) != 0))
@@ -672,7 +798,7 @@ int launch_w4a16_gemm_sk(const void* x, int64_t M, int64_t K, int64_t N, const v
                     (long long)need);
     // Buffer offsets are 32-bit: x inside one row tile, the packed weight,
     // the workspace.
-    if (total > 0x7fffffff || K > (int64_t(1) << 22) || K * nslab * kSlab / 2 >= (int64_t(1) << 31) ||
+    if (total > 0x7fffffff || K > (int64_t(1) << 22) || K * widest * kSlab / 2 >= (int64_t(1) << 31) ||
         int64_t(c.tm) * K * 2 >= (int64_t(1) << 31) || need >= (int64_t(1) << 31))
         return fail(MCV_ERR_SHAPE, "w4a16 GEMM: problem too large (M=%lld N=%lld)", (long long)M, (long long)N);
     // Each XCD takes a contiguous run of the tile order.  Down the columns,
@@ -687,7 +813,8 @@ int launch_w4a16_gemm_sk(const void* x, int64_t M, int64_t K, int64_t N, const v
     // 19.35-19.53 us along the rows, M=2048 K=3584 20.66 against 20.80-21.17,
     // M=512 K=3584 10.61 against 10.69-10.72; where x is the smaller operand
     // the column order stays ahead: M=512 K=1024 8.67 against 8.72).
-    const int64_t x_bytes = M * K * 2, w_bytes = K * N / 2 + (K / kGroup) * N * 5 / 2;
+    const int64_t cols = parts.count == 1 ? N : nslab * kSlab;
+    const int64_t x_bytes = M * K * 2, w_bytes = K * cols / 2 + (K / kGroup) * cols * 5 / 2;
     int order = c.order == 2 || (c.order == 0 && x_bytes < w_bytes) ? 1 : 0;
     if ((c.order == 3 || (c.order == 0 && x_bytes >= w_bytes)) && m_tiles >= 2) {
         // groups of g tile rows, g balancing an XCD run's x rows (g of them)
@@ -698,13 +825,29 @@ int launch_w4a16_gemm_sk(const void* x, int64_t M, int64_t K, int64_t N, const v
         order = g < 2 ? 2 : (g > m_tiles ? static_cast<int>(m_tiles) : g);
     }
     hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(total)), dim3(64 * c.nwv * c.kw), 0, stream,
-                       static_cast<const uint16_t*>(x), static_cast<const uint4*>(qw),
-                       static_cast<const uint16_t*>(scales), static_cast<const uint32_t*>(zeros),
-                       static_cast<uint32_t>(zero_bias), static_cast<uint16_t*>(out), static_cast<int>(M),
-                       static_cast<int>(K), static_cast<int>(N), static_cast<int>(nslab), static_cast<int>(m_tiles),
-                       static_cast<int>(n_tiles), c.splits, order, static_cast<uint8_t*>(ws),
-                       static_cast<uint32_t>(c.splits > 1 ? need : 0));
+                       static_cast<const uint16_t*>(x), parts, static_cast<uint16_t*>(act), static_cast<int>(M),
+                       static_cast<int>(K), static_cast<int>(m_tiles), static_cast<int>(n_tiles), c.splits, order,
+                       static_cast<uint8_t*>(ws), static_cast<uint32_t>(c.splits > 1 ? need : 0));
     return check_launch("w4a16_gemm_sk_kernel");
+}
+
+}  // namespace
+
+int launch_w4a16_gemm_sk(const void* x, int64_t M, int64_t K, int64_t N, const void* qw, const void* scales,
+                         const void* zeros, int zero_bias, void* out, const SkConfig& c, void* ws, int64_t ws_bytes,
+                         hipStream_t stream) {
+    const int64_t npad = ceil_div(N, kSlab) * kSlab;
+    W4Parts parts{};
+    parts.count = 1;
+    parts.p[0] = W4Part{static_cast<const uint4*>(qw), static_cast<const uint16_t*>(scales),
+                        static_cast<const uint32_t*>(zeros), static_cast<uint16_t*>(out), static_cast<int>(N),
+                        static_cast<int>(npad), 0, static_cast<uint32_t>(zero_bias)};
+    return launch_sk(x, M, K, parts, nullptr, false, c, ws, ws_bytes, stream);
+}
+
+int launch_w4a16_gemm_sk_parts(const void* x, int64_t M, int64_t K, const W4Parts& parts, void* act, const SkConfig& c,
+                               hipStream_t stream) {
+    return launch_sk(x, M, K, parts, act, true, c, nullptr, 0, stream);
 }
 
 }  // namespace mcv

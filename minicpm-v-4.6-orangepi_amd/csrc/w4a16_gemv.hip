@@ -22,6 +22,7 @@
 #include "argmax_exchange.h"
 #include "common.h"
 #include "gemv_body.h"
+#include "w4a16_gemm_sk.h"
 #include "w4a16_rows.h"
 
 namespace mcv {
@@ -846,9 +847,12 @@ int mcv_w4a16_gemv_multi(const void* x, int64_t M, int64_t K, const mcv_w4a16_pa
     gp.count = n_parts;
     int rc = require_device();
     if (rc != MCV_OK) return rc;
-    // a few rows: each weight widened once for all of them
+    // a few rows: each weight widened once for all of them; many: the GEMM
+    // over the concatenated column tiles (both read x in 16-byte pieces)
     const hipStream_t st = static_cast<hipStream_t>(stream);
     if (w4a16_rows_pays(M, K, total, n_parts) && w4a16_rows_ok(x, M, K, gp)) return launch_w4a16_rows(x, M, K, gp, st);
+    if (!w4a16_prefers_gemv(M, K, total * kSlab) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && w4a16_sk_fits(M, K, gp))
+        return launch_w4a16_gemm_sk_parts(x, M, K, gp, nullptr, choose_gemm(M, K, total * kSlab, false), st);
     // The k-split the smallest part would get on its own (the decode shapes
     // with K = 1024 all get 8, so the outputs equal separate launches').
     const GemvCfg cfg = choose_gemv(K / kGroup, min_slabs * M);
@@ -875,7 +879,8 @@ int mcv_w4a16_gate_up_silu(const void* x, int64_t M, int64_t K, int64_t N, const
     if (M <= 0 || M > 65535) return fail(MCV_ERR_SHAPE, "mcv_w4a16_gate_up_silu: M must be in [1, 65535] (M=%lld)", (long long)M);
     if ((rc = require_device()) != MCV_OK) return rc;
     const int64_t nslab = ceil_div(N, kSlab);
-    // a few rows as in mcv_w4a16_gemv_multi; the rule is the single weight's, so gate and up round as two mcv_w4a16_gemv calls do
+    // a few rows and many rows as mcv_w4a16_gemv_multi; the few-row rule is the
+    // single weight's, so gate and up round as two mcv_w4a16_gemv calls do
     W4Parts parts{};
     parts.count = 2;
     parts.p[0] = w4_part(qw_gate, scales_gate, zeros_gate, zero_bias_gate, N, act);
@@ -883,6 +888,8 @@ int mcv_w4a16_gate_up_silu(const void* x, int64_t M, int64_t K, int64_t N, const
     const hipStream_t st = static_cast<hipStream_t>(stream);
     if (w4a16_rows_pays(M, K, nslab, 2) && w4a16_rows_ok(x, M, K, parts))
         return launch_w4a16_rows_silu(x, M, K, parts, act, st);
+    if (!w4a16_prefers_gemv(M, K, 2 * nslab * kSlab) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && w4a16_sk_fits(M, K, parts))
+        return launch_w4a16_gemm_sk_parts(x, M, K, parts, act, choose_gemm(M, K, 2 * nslab * kSlab, false), st);
     const GemvCfg cfg = choose_gemv(K / kGroup, nslab * M);
     using Fn = void (*)(const uint16_t*, const uint4*, const uint16_t*, const uint32_t*, uint32_t, const uint4*,
                         const uint16_t*, const uint32_t*, uint32_t, uint16_t*, int, int, int);

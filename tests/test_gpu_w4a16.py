@@ -616,3 +616,33 @@ def test_several_rows_vs_oracle(mcv, oracle, cuda, M, K, N, zb):
     mag = np.abs(xf) @ np.abs(wf)
     bound = 2.0 ** -11 * np.abs(ref) + (K * 2.0 ** -24 + (2.0 ** -11 if rounded else 0)) * mag + 2.0 ** -24
     assert (np.abs(got - ref) <= bound).all(), float((np.abs(got - ref) - bound).max())
+
+
+@pytest.mark.parametrize("M,K,Ns", [(5, 1024, (3584, 512, 512)), (17, 256, (200, 72, 1000, 8)), (33, 3584, (520, 264)),
+                                    (100, 384, (1000, 72)), (300, 1024, (3584, 520)), (1100, 256, (6144, 2048))],
+                         ids=lambda v: str(v))
+def test_multi_and_gate_up_many_rows(mcv, oracle, cuda, M, K, Ns):
+    """Every part of a shared-input launch and the fused gate/up block over
+    rows that run the few-row kernel and the GEMM: fp32 sums of exact q - z."""
+    rng = np.random.default_rng(M + K + sum(Ns))
+    x = f16_normal(rng, (M, K), 1.0)
+    xf = x.view(np.float16).astype(np.float64)
+    ws, refs, mags = [], [], []
+    for i, N in enumerate(Ns):
+        _, qw, qz, sc = synth_w4a16(rng, K, N)
+        zb = i & 1
+        w = _dev_weight(mcv, qw, qz, sc)
+        ws.append(mcv.W4A16QuantizedWeight(w.qweight, w.scales, w.zeros, K, N, zb))
+        wf = (oracle.unpack_awq(qw, qz) - np.int8(zb)).astype(np.float64) * \
+            np.repeat(sc.view(np.float16).astype(np.float64), 128, axis=0)
+        refs.append(xf @ wf)
+        mags.append(np.abs(xf) @ np.abs(wf))
+    for o, ref, mag in zip(mcv.matmul_w4a16_multi(_to_dev(x), ws), refs, mags):
+        bound = 2.0 ** -11 * np.abs(ref) + K * 2.0 ** -24 * mag + 2.0 ** -24
+        assert (np.abs(_host_f32(o) - ref) <= bound).all()
+    _, qu, zu, su = synth_w4a16(rng, K, Ns[0])
+    wu = _dev_weight(mcv, qu, zu, su)
+    u = xf @ (oracle.unpack_awq(qu, zu).astype(np.float64) * np.repeat(su.view(np.float16).astype(np.float64), 128, axis=0))
+    act = _host_f32(mcv.mlp_gate_up_silu_w4a16(_to_dev(x), ws[0], wu))
+    a_o = oracle.silu_mul(oracle.f2h_rne(refs[0].astype(np.float32)), oracle.f2h_rne(u.astype(np.float32)))
+    _check(act, a_o.view(np.float16).astype(np.float32), f"gate_up M={M} K={K} N={Ns[0]}")
