@@ -143,18 +143,43 @@ __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v)
 // (one 256-thread workgroup per row; the same code in every kernel, so the
 // fused kernel is bit-identical to the two separate launches).
 
+// One step of a wave-wide butterfly without LDS: the value of lane l ^ 32 or l ^
+// 16 meets lane l's through a lane-half swap; a row rotation by R = 8, 4, 2, 1
+// then brings a lane whose value is that of lane l ^ R, since the steps before
+// made the 16-lane row periodic in 2 R.  The operands of every addition or
+// comparison, and so the result, are those of a shuffle by l ^ 32, 16, ... 1.
+template <int R>
+__device__ __forceinline__ float row_ror(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + R, 0xf, 0xf, false));
+}
+template <class Op>
+__device__ __forceinline__ float wave_butterfly(float v, Op op) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(b[0]), __uint_as_float(b[1]));
+    v = op(v, row_ror<8>(v));
+    v = op(v, row_ror<4>(v));
+    v = op(v, row_ror<2>(v));
+    return op(v, row_ror<1>(v));
+}
+
+// 1 / sqrt(tot / H + eps).
+__device__ __forceinline__ float rms_rstd(float tot, int H, float eps) {
+    return __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(tot, static_cast<float>(H)), eps)));
+}
+
 // rstd = 1 / sqrt(mean(x^2) + eps): per-thread fp32 sums of squares over the
 // strided elements i = tid, tid + 256, ... in that order (`ss`), folded by a
-// wave shuffle tree and then across the four waves in order.
+// wave butterfly and then across the four waves in order.
 __device__ __forceinline__ float block_rstd(float ss, int H, float eps) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) ss += __shfl_xor(ss, off, 64);
+    ss = wave_butterfly(ss, [](float p, float q) { return p + q; });
     __shared__ float part[4];
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = ss;
     __syncthreads();
     float tot = 0.f;
     for (int w = 0; w < static_cast<int>(blockDim.x >> 6); ++w) tot += part[w];
-    return __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn(__fdiv_rn(tot, static_cast<float>(H)), eps)));
+    return rms_rstd(tot, H, eps);
 }
 
 __device__ __forceinline__ float row_rstd(const uint16_t* __restrict__ xr, int H, float eps) {
@@ -173,11 +198,7 @@ __device__ __forceinline__ uint16_t rms_apply(uint16_t x, float rstd, uint16_t g
 
 // Workgroup maximum of per-thread |x| maxima (NaN never becomes the maximum).
 __device__ __forceinline__ float row_absmax(float m) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const float o = __shfl_xor(m, off, 64);
-        m = o > m ? o : m;
-    }
+    m = wave_butterfly(m, [](float p, float q) { return q > p ? q : p; });
     __shared__ float wmax[4];
     if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
     __syncthreads();
@@ -200,6 +221,22 @@ __device__ __forceinline__ int8_t act_quant(uint16_t x, float inv) {
     v = v < -128.0f ? -128.0f : v;
     const float r = v >= 0.0f ? __fadd_rn(v, 0.5f) : __fsub_rn(v, 0.5f);
     return static_cast<int8_t>(static_cast<int>(r));
+}
+
+// act_quant of 8 consecutive fp16 values, packed.
+__device__ __forceinline__ uint2 act_quant8(const uint4& v, float inv) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    uint32_t q[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        q[k] = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint16_t h = static_cast<uint16_t>(w[2 * k + e / 2] >> (16 * (e & 1)));
+            q[k] |= static_cast<uint32_t>(static_cast<uint8_t>(act_quant(h, inv))) << (8 * e);
+        }
+    }
+    return make_uint2(q[0], q[1]);
 }
 
 }  // namespace mcv

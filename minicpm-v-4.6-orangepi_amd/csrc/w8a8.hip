@@ -8,6 +8,7 @@
 #include <string>
 
 #include "common.h"
+#include "row_norm.h"
 
 namespace mcv {
 
@@ -33,9 +34,13 @@ namespace {
 // q = trunc(clamp(x * inv, -128, 127) +- 0.5): the closed form of
 // op_kernel/w8a8_quantize_custom.cpp:25-41 and quantized_weight.cpp:197-202,
 // every operation an explicitly rounded IEEE fp32 operation (no contraction).
-// Rows of up to 256 * PER elements are held in registers between the two
-// passes (PER = 0: strided reloads).
-template <int PER>
+// The row maximum is one in any order, so with whole aligned 16-byte chunks a
+// thread takes NC of them (VEC: chunk t + 256 c, one load and one 8-byte store
+// each); other rows of up to 256 * 16 elements are held element by element,
+// longer ones reloaded (NC = 0).  MI355X, K=3584, 2-byte loads and 1-byte stores
+// against chunks: M=1 3.1 / 2.3 us, M=40 3.4 / 2.6, M=3000 10.0 / 9.0 (a wave per
+// row instead of four: 9.9).
+template <int NC, bool VEC>
 __global__ __launch_bounds__(256) void w8a8_quant_act_kernel(const uint16_t* __restrict__ x, int K,
                                                              int8_t* __restrict__ xq, float* __restrict__ s32,
                                                              uint16_t* __restrict__ s16) {
@@ -45,13 +50,35 @@ __global__ __launch_bounds__(256) void w8a8_quant_act_kernel(const uint16_t* __r
     int8_t* qr = xq + static_cast<size_t>(row) * K;
     float m = 0.f;
     float scale;
-    if constexpr (PER > 0) {
+    if constexpr (VEC && NC > 0) {
+        uint4 xv[NC];
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const int i = 8 * (t + 256 * c);
+            xv[c] = i < K ? *reinterpret_cast<const uint4*>(xr + i) : make_uint4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float v = fabsf(h2f(chunk_get(xv[c], e)));  // padding contributes 0, never above the max
+                m = v > m ? v : m;
+            }
+        scale = act_scale(row_absmax(m));
+        const float inv = __fdiv_rn(1.0f, scale);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const int i = 8 * (t + 256 * c);
+            if (i < K) *reinterpret_cast<uint2*>(qr + i) = act_quant8(xv[c], inv);
+        }
+    } else if constexpr (NC > 0) {
+        constexpr int PER = 8 * NC;
         uint16_t xv[PER];
 #pragma unroll
         for (int j = 0; j < PER; ++j) xv[j] = t + 256 * j < K ? xr[t + 256 * j] : uint16_t(0);
 #pragma unroll
         for (int j = 0; j < PER; ++j) {
-            const float v = fabsf(h2f(xv[j]));                // padding contributes 0, never above the max
+            const float v = fabsf(h2f(xv[j]));
             m = v > m ? v : m;
         }
         scale = act_scale(row_absmax(m));
@@ -67,79 +94,6 @@ __global__ __launch_bounds__(256) void w8a8_quant_act_kernel(const uint16_t* __r
         scale = act_scale(row_absmax(m));
         const float inv = __fdiv_rn(1.0f, scale);
         for (int k = t; k < K; k += blockDim.x) qr[k] = act_quant(xr[k], inv);
-    }
-    if (t == 0) {
-        if (s32) s32[row] = scale;
-        if (s16) s16[row] = f2h(scale);
-    }
-}
-
-// RMSNorm and the activation quantisation in one pass over a row (the decode
-// sequence rms_norm -> w8a8_quantize of decoder_layer.cpp:955-966,
-// 1022-1032): the normed fp16 row is formed once, optionally stored (the
-// other projections of the step still read it), and quantised from the same
-// fp16 values -- bit-identical to rms_norm_kernel + w8a8_quant_act_kernel
-// (same element order per thread, same reductions).  Rows of up to 256 * PER
-// elements stay in registers, x and gamma loaded together up front; longer
-// rows take the strided loops (PER = 0).
-template <int PER>
-__global__ __launch_bounds__(256) void rms_norm_quant_kernel(const uint16_t* __restrict__ x,
-                                                             const uint16_t* __restrict__ gamma, int H, float eps,
-                                                             uint16_t* __restrict__ normed, int8_t* __restrict__ xq,
-                                                             float* __restrict__ s32, uint16_t* __restrict__ s16) {
-    const int row = blockIdx.x;
-    const int t = threadIdx.x;
-    const uint16_t* xr = x + static_cast<size_t>(row) * H;
-    uint16_t* nr = normed ? normed + static_cast<size_t>(row) * H : nullptr;
-    int8_t* qr = xq + static_cast<size_t>(row) * H;
-    float m = 0.f;
-    float inv;
-    float scale;
-    if constexpr (PER > 0) {
-        uint16_t xv[PER], gv[PER];
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const int i = t + 256 * j;
-            xv[j] = i < H ? xr[i] : uint16_t(0);
-            gv[j] = i < H ? gamma[i] : uint16_t(0);
-        }
-        float ss = 0.f;
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            if (t + 256 * j < H) {
-                const float v = h2f(xv[j]);
-                ss = fmaf(v, v, ss);
-            }
-        }
-        const float rstd = block_rstd(ss, H, eps);
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const int i = t + 256 * j;
-            if (i < H) {
-                xv[j] = rms_apply(xv[j], rstd, gv[j]);                  // xv now holds the normed row
-                if (nr) nr[i] = xv[j];
-                const float v = fabsf(h2f(xv[j]));
-                m = v > m ? v : m;
-            }
-        }
-        scale = act_scale(row_absmax(m));
-        inv = __fdiv_rn(1.0f, scale);
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const int i = t + 256 * j;
-            if (i < H) qr[i] = act_quant(xv[j], inv);
-        }
-    } else {
-        const float rstd = row_rstd(xr, H, eps);
-        for (int i = t; i < H; i += blockDim.x) {
-            const uint16_t h = rms_apply(xr[i], rstd, gamma[i]);
-            if (nr) nr[i] = h;
-            const float v = fabsf(h2f(h));
-            m = v > m ? v : m;
-        }
-        scale = act_scale(row_absmax(m));
-        inv = __fdiv_rn(1.0f, scale);
-        for (int i = t; i < H; i += blockDim.x) qr[i] = act_quant(rms_apply(xr[i], rstd, gamma[i]), inv);
     }
     if (t == 0) {
         if (s32) s32[row] = scale;
@@ -368,7 +322,14 @@ int mcv_w8a8_quantize_act(const void* x, int64_t M, int64_t K, int8_t* xq, float
         return fail(MCV_ERR_SHAPE, "w8a8_quantize: bad shape M=%lld K=%lld", (long long)M, (long long)K);
     int rc = require_device();
     if (rc != MCV_OK) return rc;
-    auto fn = K <= 1024 ? w8a8_quant_act_kernel<4> : K <= 4096 ? w8a8_quant_act_kernel<16> : w8a8_quant_act_kernel<0>;
+    const bool vec = K % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(xq) % 8 == 0;
+    auto fn = vec ? (K <= 2048   ? w8a8_quant_act_kernel<1, true>
+                     : K <= 4096 ? w8a8_quant_act_kernel<2, true>
+                     : K <= 8192 ? w8a8_quant_act_kernel<4, true>
+                                 : w8a8_quant_act_kernel<0, false>)
+                  : (K <= 2048   ? w8a8_quant_act_kernel<1, false>
+                     : K <= 4096 ? w8a8_quant_act_kernel<2, false>
+                                 : w8a8_quant_act_kernel<0, false>);
     hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(M)), dim3(256), 0, static_cast<hipStream_t>(stream),
                        static_cast<const uint16_t*>(x), static_cast<int>(K), xq, s32, static_cast<uint16_t*>(s16));
     return check_launch("w8a8_quant_act_kernel");
@@ -381,11 +342,10 @@ int mcv_rms_norm_w8a8_quantize(const void* x, const void* gamma, int64_t M, int6
         return fail(MCV_ERR_SHAPE, "rms_norm_w8a8_quantize: bad shape M=%lld H=%lld or eps", (long long)M, (long long)H);
     int rc = require_device();
     if (rc != MCV_OK) return rc;
-    auto fn = H <= 1024 ? rms_norm_quant_kernel<4> : H <= 4096 ? rms_norm_quant_kernel<16> : rms_norm_quant_kernel<0>;
-    hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(M)), dim3(256), 0, static_cast<hipStream_t>(stream),
-                       static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(gamma), static_cast<int>(H),
-                       static_cast<float>(eps), static_cast<uint16_t*>(normed), xq, s32, static_cast<uint16_t*>(s16));
-    return check_launch("rms_norm_quant_kernel");
+    launch_rms<true>(static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(gamma), M, H, static_cast<float>(eps),
+                     static_cast<uint16_t*>(normed), xq, s32, static_cast<uint16_t*>(s16),
+                     static_cast<hipStream_t>(stream));
+    return check_launch("rms_row_kernel<quantise>");
 }
 
 int mcv_w8a8_gemm_i32(const int8_t* xq, int64_t M, int64_t K, int64_t N, const int8_t* w, int w_layout, int32_t* acc,

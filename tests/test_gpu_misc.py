@@ -111,3 +111,35 @@ def test_rms_norm_w8a8_quantize_fused(mcv, oracle, cuda, M, H):
     # without the fp16 row
     none, xq2, xs2, _ = mcv.rms_norm_w8a8_quantize(xd, gd, 1e-6, want_normed=False)
     assert none is None and torch.equal(xq2, xq) and torch.equal(xs2, xs)
+
+
+# The row kernels at the edges of their register and chunk variants: rows of
+# whole aligned 16-byte chunks and ragged ones, one and two chunks a thread,
+# rows longer than a workgroup holds, and rms_norm onto its own input.
+@pytest.mark.parametrize("M,H", [(2, 8), (3, 256), (2, 257), (5, 1024), (2, 2056), (600, 1032), (2, 4104), (2, 8192),
+                                 (2, 8200), (1, 8191)])
+def test_row_kernels_edges(mcv, oracle, cuda, M, H):
+    torch = _torch()
+    rng = np.random.default_rng(7 * M + H)
+    x, gamma = f16_normal(rng, (M, H), 1.5), f16_normal(rng, (H,), 1.0)
+    xd, gd = _f16_dev(x), _f16_dev(gamma)
+    want = mcv.rms_norm(xd, gd, 1e-6)
+    ref = oracle.rms_norm(x, gamma, 1e-6).astype(np.int64)
+    got = _u16(want).astype(np.int64)
+    assert np.abs(got - ref).max() <= 1                  # an fp16 ulp: the sum's order
+    normed, xq, xs, _ = mcv.rms_norm_w8a8_quantize(xd, gd, 1e-6)
+    q, s, _ = mcv.w8a8_quantize(want)
+    assert torch.equal(normed, want) and torch.equal(xq, q) and torch.equal(xs, s)
+    oq, os32, _ = oracle.w8a8_quantize_act(_u16(want))
+    assert (q.cpu().numpy() == oq).all() and (s.cpu().numpy() == os32).all()
+    inplace = xd.clone()
+    assert torch.equal(mcv.rms_norm(inplace, gd, 1e-6, out=inplace), want)
+
+
+@pytest.mark.parametrize("n,off", [((1 << 21) + 5, 0), ((1 << 21) + 9, 1)])
+def test_silu_mul_chunks(mcv, oracle, cuda, n, off):
+    rng = np.random.default_rng(n)
+    g, u = f16_normal(rng, (n,), 3.0), f16_normal(rng, (n,), 1.0)
+    out = mcv.silu_mul(_f16_dev(g)[off:], _f16_dev(u)[off:])
+    got = _u16(out).astype(np.int64)
+    assert np.abs(got - oracle.silu_mul(g[off:], u[off:]).astype(np.int64)).max() <= 1
