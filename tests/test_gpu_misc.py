@@ -143,3 +143,21 @@ def test_silu_mul_chunks(mcv, oracle, cuda, n, off):
     out = mcv.silu_mul(_f16_dev(g)[off:], _f16_dev(u)[off:])
     got = _u16(out).astype(np.int64)
     assert np.abs(got - oracle.silu_mul(g[off:], u[off:]).astype(np.int64)).max() <= 1
+
+
+# Rows cut into parts over workgroups: a part's and a chunk's borders, ties
+# between parts, the values that cannot win, a row with no candidate.
+@pytest.mark.parametrize("M,N", [(1, 65536), (3, 131073), (40, 70001), (300, 65541)])
+def test_argmax_split_rows(mcv, oracle, cuda, M, N):
+    rng = np.random.default_rng(M + N)
+    x = rng.integers(0, 65536, (M, N), dtype=np.uint16)                  # every bit pattern: NaN, inf, subnormals
+    x[(x & 0x7FFF) == 0x7C00] = 0x3C00
+    x[0, [0, N // 3, N - 1]] = 0x7C00                                    # +inf in the first, a middle and the last part
+    if M > 2:
+        x[1] = (x[1] & 0x83FF) | (rng.integers(0, 2, N, dtype=np.uint16) << 15)      # zeros and subnormals: index 0
+        x[2] = 0xFE01
+        x[2, N - 1] = 0xFBFF                                             # -65504 alone among NaN
+    if M > 3:
+        x[3] = 0xFC00                                                    # all -inf: 0
+    got = mcv.argmax_last_dim(_f16_dev(x)).cpu().numpy()
+    assert got.tolist() == [oracle.argmax_f16(x[m]) for m in range(M)]
