@@ -10,7 +10,8 @@
 // both operands in LDS (w8a8_gemm_lds.hip); this file holds the layout's
 // GEMV and the dispatch.
 //
-// GEMV (M <= 4, or M <= 2 when K > 2048): one workgroup per slab, waves splitting K, v_dot4
+// GEMV (M <= 2, where the few-row kernels of w8a8_rows.hip do not take over, and
+// the fused gate + up to M = 4): one workgroup per slab, waves splitting K, v_dot4
 // int8 dot products on the same operand lines, partial sums meeting in LDS.
 //
 // Replaces matmul_w8a8_i32_custom + w8a8_dequant_custom and their host
@@ -392,8 +393,13 @@ int64_t w8a8_tiled_bytes(int64_t K, int64_t N) {
 int launch_w8a8_gemm_lds(const int8_t* xq, int64_t M, int64_t K, int64_t N, const int8_t* w, void* out, bool f16,
                          const void* xs, int xs16, const void* ws, int ws16, hipStream_t stream);
 std::string w8a8_gemm_lds_name(int64_t M, int64_t N, bool f16);
+bool w8a8_uses_rows(int64_t M, int64_t K, int64_t N);
+std::string w8a8_rows_name(int64_t M, int64_t K, int64_t N, bool f16);
+int launch_w8a8_rows(const int8_t* xq, int64_t M, int64_t K, int64_t N, const int8_t* w, void* out, bool f16,
+                     const void* xs, int xs16, const void* ws, int ws16, hipStream_t stream);
 
-// The GEMV takes M <= 4, and M <= 2 past K = 2048 (launch_w8a8_tiled).
+// Of what the few-row kernels leave, the GEMV takes M <= 4, and M <= 2 past K =
+// 2048 (launch_w8a8_tiled).
 bool w8a8_uses_gemv(int64_t M, int64_t K) {
     const int64_t KB = ceil_div(K, 128) * 4;
     return M <= 2 || (M <= 4 && KB <= 64);
@@ -401,6 +407,7 @@ bool w8a8_uses_gemv(int64_t M, int64_t K) {
 
 // The kernel launch_w8a8_tiled runs for M x K x N, as text (report labels).
 std::string w8a8_tiled_name(int64_t M, int64_t K, int64_t N, bool f16) {
+    if (w8a8_uses_rows(M, K, N)) return w8a8_rows_name(M, K, N, f16);
     if (!w8a8_uses_gemv(M, K)) return w8a8_gemm_lds_name(M, N, f16);
     const int64_t nslab = ceil_div(N, kSlab), KB = ceil_div(K, 128) * 4;
     const bool narrow = nslab < 128;
@@ -420,6 +427,7 @@ int launch_w8a8_tiled(const int8_t* xq, int64_t M, int64_t K, int64_t N, const i
     const int64_t KB = ceil_div(K, 128) * 4;            // 32-k blocks per slab (padded to whole stages)
     if (nslab * KB * 2 * kW8Block >= (int64_t(1) << 32) || M * K >= (int64_t(1) << 32))
         return fail(MCV_ERR_SHAPE, "w8a8 tiled: weight or activation exceeds 4 GiB");
+    if (w8a8_uses_rows(M, K, N)) return launch_w8a8_rows(xq, M, K, N, w, out, f16, xs, xs16, ws, ws16, stream);
     // The GEMV up to M = 4, but only up to M = 2 past K = 2048, where its
     // serial k-blocks per wave cost more than the GEMM's fixed start
     // (MI355X, graph-replayed, us: K=3584 N=1024 GEMV M=1/2/4 4.8/6.3/8.4,

@@ -538,3 +538,26 @@ def test_lm_head_w8a8_one_launch_graph_replays(mcv, cuda):
         assert int(tok.item()) == want, f"replay {i}"
         assert torch.equal(logits.view(torch.int16), want_logits.view(torch.int16)), f"replay {i}"
     assert int(ws[:4].view(torch.int32).item()) == 0         # no wait gave up
+
+
+# The few-row kernels at the edges of their 16-row blocks, of the waves' trips
+# over K (13 chunks of 16, 40 groups) and of the wide kernel's column units,
+# ragged N: int32 and the fused fp16 epilogue bit-exact.
+@pytest.mark.parametrize("M,K,N", [(1, 2064, 72), (2, 3584, 1024), (3, 208, 80), (16, 1024, 3584), (17, 5008, 200),
+                                   (33, 2048, 1000), (64, 3584, 1003), (65, 3584, 1000), (200, 2064, 520),
+                                   (5, 256, 128100), (32, 144, 57601), (40, 128, 76801)], ids=lambda v: str(v))
+def test_few_rows_bit_exact(mcv, oracle, cuda, M, K, N):
+    torch = _torch()
+    rng = np.random.default_rng(M + K + N)
+    xq = rng.integers(-128, 128, (M, K), dtype=np.int8)
+    wq = rng.integers(-127, 128, (K, N), dtype=np.int8)
+    xs, ws = rng.random(M, dtype=np.float32) * 1e-2, rng.random(N, dtype=np.float32) * 1e-3
+    w = mcv.W8A8QuantizedWeight(torch.from_numpy(mcv.pack_w8a8_tiled(wq)).cuda(), torch.from_numpy(ws).cuda().half(),
+                                torch.from_numpy(ws).cuda(), K, N, mcv.W8_TILED)
+    xd, sd = torch.from_numpy(xq).cuda(), torch.from_numpy(xs).cuda()
+    acc = mcv.matmul_w8a8_i32(xd, w)
+    assert "rows" in mcv.lib().mcv_w8a8_gemm_kernel_name(M, K, N, mcv.W8_TILED, 1).decode()
+    ref = oracle.gemm_i32(xq, wq)
+    assert (acc.cpu().numpy() == ref).all()
+    assert torch.equal(mcv.matmul_w8a8(xd, sd, w), mcv.w8a8_dequant(acc, sd, w.w_scale_f32))
+    assert torch.equal(mcv.matmul_w8a8(xd, sd.half(), w, use_f32_scale=False), mcv.w8a8_dequant(acc, sd.half(), w.w_scale))
