@@ -30,7 +30,9 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
 // Greedy argmax of fp16 rows, first maximum, with argmax_key16's order: NaN and
 // -inf never win, subnormals and -0 count as +0.
 //
-// A row is read in 16-byte chunks of eight values, four in flight per lane.
+// One workgroup of 1024 threads per row, read in 16-byte chunks of eight values,
+// four in flight per lane (eight: rows of 31012 4.9 us against 4.1, longer ones the
+// same).
 // What bounds it is the VALU work per value, so a chunk is compared as a whole:
 // packed 16-bit integer steps map a value to a signed order (rank16) in which
 // every value that cannot win sits below kRankNone, a packed maximum folds the
@@ -40,9 +42,10 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
 // replaces).  At most seven values up to the first 16-byte boundary and after
 // the last chunk go one by one.  The lanes' 64-bit keys (value, then lowest
 // index) meet through wave shuffles and LDS.  MI355X, rows of 248094: building
-// argmax_key16 per value took 31 us in one workgroup; one
-// row is now 7.1 us, 6 rows 8.7, 32 rows 12.1 (split over workgroups, below), and
-// rows of 31012 in one workgroup each 6.4 -> 4.1.
+// argmax_key16 per value took 31 us; chunks 10.3, 6
+// rows 10.5, 32 rows 11.0, 6 rows of 31012 6.4 -> 4.1.  Cutting a row over
+// workgroups whose keys meet by atomic maximum takes two more launches: 7.1 us
+// for one row, 8.7 for 6, 12.1 for 32, and ~6 us more of the host.
 
 // The order-preserving rank of two packed fp16 values: sign-magnitude to two's
 // complement, then + 0x3ff, which wraps positive NaN (above +inf) around to the
@@ -66,34 +69,31 @@ __device__ __forceinline__ int rank_max8(const uint4& q) {
     return rank_flush(m[0] > m[1] ? m[0] : m[1]);
 }
 
-// Row blockIdx.y of [M][N], part blockIdx.x of gridDim.x of its chunks.  SPLIT:
-// the part's key goes into the row's word of `idx` by atomic maximum (zeroed
-// before, turned into the index after this launch); else the row's index.
-template <int T, bool SPLIT>
-__global__ __launch_bounds__(T) void argmax_kernel(const uint16_t* __restrict__ x, int64_t N, int64_t* __restrict__ idx) {
-    const uint16_t* xr = x + static_cast<size_t>(blockIdx.y) * N;
+constexpr int kArgThreads = 1024;
+__global__ __launch_bounds__(kArgThreads) void argmax_kernel(const uint16_t* __restrict__ x, int64_t N,
+                                                             int64_t* __restrict__ idx) {
+    const uint16_t* xr = x + static_cast<size_t>(blockIdx.x) * N;
     const int tid = threadIdx.x;
     const int64_t head64 = static_cast<int64_t>((16u - (reinterpret_cast<uintptr_t>(xr) & 15u)) & 15u) / 2;
     const int64_t head = head64 < N ? head64 : N;
     const uint4* __restrict__ v = reinterpret_cast<const uint4*>(xr + head);
     const int64_t nv = (N - head) / 8;
-    const int64_t c0 = SPLIT ? nv * blockIdx.x / gridDim.x : 0, c1 = SPLIT ? nv * (blockIdx.x + 1) / gridDim.x : nv;
     int br = kRankNone;                          // best rank so far and its first chunk
     int64_t bc = 0;
     constexpr int U = 4;
-    for (int64_t j0 = c0 + tid; j0 < c1; j0 += int64_t(T) * U) {
+    for (int64_t j0 = tid; j0 < nv; j0 += int64_t(kArgThreads) * U) {
         uint4 q[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {            // past the end: -inf, never a candidate
-            const int64_t j = j0 + int64_t(u) * T;
-            q[u] = j < c1 ? v[j] : make_uint4(0xfc00fc00u, 0xfc00fc00u, 0xfc00fc00u, 0xfc00fc00u);
+            const int64_t j = j0 + int64_t(u) * kArgThreads;
+            q[u] = j < nv ? v[j] : make_uint4(0xfc00fc00u, 0xfc00fc00u, 0xfc00fc00u, 0xfc00fc00u);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int r = rank_max8(q[u]);
             const bool take = r > br;
             br = take ? r : br;
-            bc = take ? j0 + int64_t(u) * T : bc;
+            bc = take ? j0 + int64_t(u) * kArgThreads : bc;
         }
     }
     unsigned long long best = 0ull;
@@ -109,29 +109,16 @@ __global__ __launch_bounds__(T) void argmax_kernel(const uint16_t* __restrict__ 
         for (int e = 7; e >= 0; --e) first = rank_flush(rank16(w[e / 2])[e & 1]) == br ? e : first;
         visit(head + 8 * bc + first);
     }
-    if ((!SPLIT || blockIdx.x == 0) && tid < head) visit(tid);
-    if ((!SPLIT || blockIdx.x == gridDim.x - 1) && head + 8 * nv + tid < N) visit(head + 8 * nv + tid);
+    if (tid < head) visit(tid);
+    if (head + 8 * nv + tid < N) visit(head + 8 * nv + tid);
     best = wave_max_u64(best);
-    __shared__ unsigned long long wbest[T / 64];
+    __shared__ unsigned long long wbest[kArgThreads / 64];
     if ((tid & 63) == 0) wbest[tid >> 6] = best;
     __syncthreads();
     if (tid < 64) {
-        best = wave_max_u64(tid < T / 64 ? wbest[tid] : 0ull);
-        if (tid == 0) {
-            if constexpr (SPLIT) {
-                if (best != 0ull) atomicMax(reinterpret_cast<unsigned long long*>(idx) + blockIdx.y, best);
-            } else {
-                idx[blockIdx.y] = argmax_index(best);
-            }
-        }
+        best = wave_max_u64(tid < kArgThreads / 64 ? wbest[tid] : 0ull);
+        if (tid == 0) idx[blockIdx.x] = argmax_index(best);
     }
-}
-
-// DONE = false: zeroes the rows' key words; true: turns them into indices.
-template <bool DONE>
-__global__ __launch_bounds__(256) void argmax_keys_kernel(int64_t* __restrict__ idx, int64_t M) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i < M) idx[i] = DONE ? argmax_index(static_cast<unsigned long long>(idx[i])) : 0;
 }
 
 }  // namespace
@@ -163,25 +150,8 @@ int mcv_argmax_f16(const void* x, int64_t M, int64_t N, int64_t* idx, mcv_stream
         return fail(MCV_ERR_SHAPE, "argmax: bad shape M=%lld N=%lld", (long long)M, (long long)N);
     int rc = require_device();
     if (rc != MCV_OK) return rc;
-    const hipStream_t st = static_cast<hipStream_t>(stream);
-    const uint16_t* xp = static_cast<const uint16_t*>(x);
-    // Long rows that one workgroup each would leave most CUs idle are cut into
-    // parts of at least 1024 chunks, about four workgroups per CU in all; the
-    // two launches around them cost ~3.5 us, which rows below 64K do not pay.
-    const int64_t parts = ceil_div(1024, M) < N / 8192 ? ceil_div(1024, M) : N / 8192;
-    if (N >= 65536 && M <= 512 && parts > 1) {
-        const dim3 words(static_cast<unsigned>(ceil_div(M, 256)));
-        hipLaunchKernelGGL(argmax_keys_kernel<false>, words, dim3(256), 0, st, idx, M);
-        hipLaunchKernelGGL((argmax_kernel<256, true>), dim3(static_cast<unsigned>(parts), static_cast<unsigned>(M)), dim3(256),
-                           0, st, xp, N, idx);
-        hipLaunchKernelGGL(argmax_keys_kernel<true>, words, dim3(256), 0, st, idx, M);
-        return check_launch("argmax_kernel<split>");
-    }
-    for (int64_t m0 = 0; m0 < M; m0 += 65535) {  // rows are the grid's y
-        const int64_t rows = M - m0 < 65535 ? M - m0 : 65535;
-        hipLaunchKernelGGL((argmax_kernel<1024, false>), dim3(1, static_cast<unsigned>(rows)), dim3(1024), 0, st, xp + m0 * N,
-                           N, idx + m0);
-    }
+    hipLaunchKernelGGL(argmax_kernel, dim3(static_cast<unsigned>(M)), dim3(kArgThreads), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const uint16_t*>(x), N, idx);
     return check_launch("argmax_kernel");
 }
 

@@ -145,14 +145,14 @@ def test_silu_mul_chunks(mcv, oracle, cuda, n, off):
     assert np.abs(got - oracle.silu_mul(g[off:], u[off:]).astype(np.int64)).max() <= 1
 
 
-# Rows cut into parts over workgroups: a part's and a chunk's borders, ties
-# between parts, the values that cannot win, a row with no candidate.
+# Long rows: ties between lanes and chunks, the values that cannot win in every
+# bit pattern, a row with no candidate.
 @pytest.mark.parametrize("M,N", [(1, 65536), (3, 131073), (40, 70001), (300, 65541)])
-def test_argmax_split_rows(mcv, oracle, cuda, M, N):
+def test_argmax_long_rows(mcv, oracle, cuda, M, N):
     rng = np.random.default_rng(M + N)
     x = rng.integers(0, 65536, (M, N), dtype=np.uint16)                  # every bit pattern: NaN, inf, subnormals
     x[(x & 0x7FFF) == 0x7C00] = 0x3C00
-    x[0, [0, N // 3, N - 1]] = 0x7C00                                    # +inf in the first, a middle and the last part
+    x[0, [0, N // 3, N - 1]] = 0x7C00                                    # +inf in the first, a middle and the last chunk
     if M > 2:
         x[1] = (x[1] & 0x83FF) | (rng.integers(0, 2, N, dtype=np.uint16) << 15)      # zeros and subnormals: index 0
         x[2] = 0xFE01
