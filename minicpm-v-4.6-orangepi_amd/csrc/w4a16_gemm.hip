@@ -32,8 +32,14 @@ bool small_output(int64_t M, int64_t N) { return M >= 1 && (M < 8 || M * N < 655
 
 // The GEMM's configuration for M x K x N.  First the largest tile whose grid
 // gives 200-256 workgroups, one tile each (a workgroup per CU): 128 x 256
-// (eight waves), 64 x 128, 64 x 64, 32 x 128, 32 x 64; past 256, the largest
-// that reaches 200 other than 64 x 64.  Failing that (few rows and N =
+// (eight waves), 64 x 128, 64 x 64, 32 x 128, 32 x 64; past 256
+// tiles of even the smallest, the least of a cost table: what a CU's tiles take
+// depends on how many it gets (a shape just past 256 takes two rounds) and on
+// whether another workgroup on the CU covers a tile's start and end.  Against
+// the largest tile that reached 200 workgroups, us: M=8192 K=1024 N=3584 65.2 ->
+// 61.8 (128 x 128, two per CU), M=1100 K=1024 N=8192 30.3 -> 24.9 and N=3584 15.6
+// -> 12.1, M=577 N=8192 21.2 -> 15.9, M=1600 N=3584 22.5 -> 16.6, M=1100 K=3584
+// N=1024 22.2 -> 15.5, M=4096 37.2 -> 32.9.  Failing that (few rows and N =
 // 1024-like widths), with a workspace, K is split across workgroups on 32 x 64
 // tiles: the most ways that keep the grid within one workgroup per CU and
 // leave each workgroup at least 7 quantisation groups on average (splits are
@@ -67,7 +73,24 @@ bool small_output(int64_t M, int64_t N) { return M >= 1 && (M < 8 || M * N < 655
 // (3584, 1024), (1024, 6144), (1024, 2048), (2048, 1024): 10-25 % faster
 // where it changes the configuration, except 0.05-0.15 us slower where its
 // grid passes 256 workgroups (M = 96-192 at N = 3584-6144).
-SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split) {
+SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split, bool exact) {
+    // us per quantisation group of K with n tiles on the fullest CU, n = 1, 2 and
+    // each further one, fitted to sweeps at M = 300..8192, N = 1024..8192, K = 1024,
+    // 2048 and 3584 (a call adds ~3 us): MI355X.
+    struct Cost {
+        SkConfig c;
+        double one, two, more;
+    };
+    static const Cost kCosts[] = {
+        {{128, 8, 3, 1}, 1.85, 3.8, 2.1},                      // 128 x 256
+        {{128, 4, 2, 1, 1, 1, 1}, 1.17, 1.85, 1.05},           // 128 x 128, two workgroups per CU
+        {{128, 4, 3, 1, 1, 1, 0}, 1.15, 2.25, 1.1},            // 128 x 128 through LDS
+        {{64, 4, 2, 1, 1, 1, 1}, 0.8, 1.2, 0.6},               // 64 x 128, three
+        {{64, 4, 3, 1}, 0.6, 1.2, 0.75},                       // 64 x 128, two k-parts
+        {{64, 2, 3, 1}, 0.42, 0.75, 0.4},                      // 64 x 64
+        {{32, 4, 3, 1}, 0.42, 0.65, 0.55},                     // 32 x 128
+        {{32, 2, 3, 1}, 0.3, 0.47, 0.27},                      // 32 x 64
+    };
     constexpr SkConfig kOne[] = {{128, 8, 3, 1}, {64, 4, 3, 1}, {64, 2, 3, 1}, {32, 4, 3, 1}, {32, 2, 3, 1}};
     const int64_t G = K / kGroup;
     auto finish = [&](SkConfig c) {
@@ -77,17 +100,31 @@ SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split) {
         return c;
     };
     // one tile per workgroup and one workgroup per CU where a tile fits that
-    // (200-256 tiles); else the largest tile that still covers most CUs,
-    // 64 x 64 aside (past 256 tiles it trails 32 x 128 by 5-20 %)
+    // (200-256 tiles); exact operands (several weights) leave the 128 x 256 tile
+    // out, whose registers they fill (gate + up M=1100 21.4 us and here 21.4-21.9, qkv + z 30.1 and 26.3)
     for (const SkConfig& c : kOne) {
+        if (exact && c.nwv == 8) continue;
         const int64_t t = w4a16_sk_tiles(M, N, c);
         if (t >= 200 && t <= 256) return finish(c);
     }
-    for (const SkConfig& c : kOne)
-        if (w4a16_sk_tiles(M, N, c) >= 200 && !(c.tm == 64 && c.nwv == 2)) return finish(c);
     SkConfig c{32, 2, 3, 1};
     const int64_t tiles = w4a16_sk_tiles(M, N, c);
-    if (!can_split || tiles > kSkMaxSplitTiles) return finish(c);
+    if (tiles > 256) {
+        SkConfig best = c;
+        double least = 0;
+        for (const Cost& k : kCosts) {
+            if (exact && k.c.nwv == 8) continue;
+            const int64_t n = ceil_div(w4a16_sk_tiles(M, N, k.c), 256);
+            const double t = n == 1 ? k.one : k.two + static_cast<double>(n - 2) * k.more;
+            if (least == 0 || t < least) {
+                least = t;
+                best = k.c;
+            }
+        }
+        // the 128 x 128 and three-per-CU shapes are what the table says
+        return best.ns == 2 || (best.tm == 128 && best.nwv == 4) ? best : finish(best);
+    }
+    if (!can_split) return finish(c);
     // the K split: the most ways within 256 workgroups that leave at least 7
     // groups per workgroup on average, cut in whole stages (two groups each
     // where K/128 is even)

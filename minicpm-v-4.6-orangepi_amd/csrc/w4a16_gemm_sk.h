@@ -48,8 +48,9 @@ int launch_w4a16_gemm_sk_parts(const void* x, int64_t M, int64_t K, const W4Part
                                hipStream_t stream);
 // True where the GEMM's 32-bit buffer offsets cover this call.
 bool w4a16_sk_fits(int64_t M, int64_t K, const W4Parts& parts);
-// The configuration the dispatch (w4a16_gemm.hip) takes for M x K x N.
-SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split);
+// The configuration the dispatch (w4a16_gemm.hip) takes for M x K x N; `exact`:
+// for launch_w4a16_gemm_sk_parts.
+SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split, bool exact = false);
 bool w4a16_prefers_gemv(int64_t M, int64_t K, int64_t N);
 
 }  // namespace mcv

@@ -55,6 +55,11 @@
 // MI355X this measured 0-9 % faster on 64- and 32-row tiles and the same on
 // 128 x 256 (whose LDS path stays).
 //
+// NS = 2 (WR = 1): a stage buffer less, so that two workgroups (64-row tiles:
+// three) share a CU.  One tile's first loads, barriers and output then overlap
+// another's MFMAs, which a single 128 x 256 tile per CU leaves exposed (choose_gemm
+// has the figures).
+//
 // K split (S > 1): workgroup (tile, p) runs the stages [p U/S, (p+1) U/S)
 // of the U = G/KG stages over K (S need not divide U).
 // Each writes its fp32 partial tile (after the k-parts' sum) to the
@@ -174,7 +179,7 @@ struct CfgS {
 // same output columns, and the epilogue combines the two halves of the staged
 // fp16 tile -- the roundings of two launches and silu_mul.
 template <int TM, int NWV, int NS, int KG, int KW, int WR, int KIND, int EX>
-__global__ __launch_bounds__(64 * NWV * KW) void w4a16_gemm_sk_kernel(
+__global__ __launch_bounds__(64 * NWV * KW, NS == 2 && KW == 1 ? 2 : 1) void w4a16_gemm_sk_kernel(
     const uint16_t* __restrict__ x, W4Parts parts, uint16_t* __restrict__ act, int M, int K, int m_tiles, int n_tiles,
     int S, int order, uint8_t* __restrict__ ws, uint32_t ws_bytes) {
     using C = CfgS<TM, NWV, NS, KG, KW, WR, EX>;
@@ -711,7 +716,7 @@ using SkFn = void (*)(const uint16_t*, W4Parts, uint16_t*, int, int, int, int, i
     X(64, 4, 3, 2, 1, 0) X(32, 4, 3, 2, 1, 0) X(64, 4, 3, 2, 2, 0) X(32, 4, 3, 2, 2, 0) X(128, 8, 4, 1, 1, 1)   \
     X(64, 4, 3, 1, 1, 1) X(64, 4, 3, 2, 2, 1) X(64, 4, 4, 2, 2, 1) X(32, 4, 3, 1, 1, 1) X(32, 4, 3, 2, 1, 1)   \
     X(32, 4, 3, 2, 2, 1) X(32, 2, 3, 1, 1, 1) X(32, 2, 3, 2, 2, 1) X(64, 2, 3, 2, 2, 1) X(32, 2, 4, 2, 2, 1)   \
-    X(128, 2, 3, 1, 1, 1) X(128, 2, 2, 2, 2, 1) X(64, 2, 3, 1, 1, 1)
+    X(128, 2, 3, 1, 1, 1) X(128, 2, 2, 2, 2, 1) X(64, 2, 3, 1, 1, 1) X(128, 4, 2, 1, 1, 1) X(64, 4, 2, 1, 1, 1)
 // EX for one weight: where it is at least as fast.  MI355X, us, EX / rounded
 // weights: 32 x 64 M=128 K=3584 7.81 / 8.01, 32 x 128 M=1100 K=3584 19.7 / 21.0,
 // 64 x 128 M=1100 N=3584 16.07 / 16.35; but 128 x 256 (twice the accumulators)
@@ -721,7 +726,8 @@ constexpr int one_exact(int tm, int nwv, int, int, int, int) { return tm == 32 |
 // what the dispatch picks (choose_gemm), for several weights
 #define MCV_SK_PARTS_SHAPES(X)                                                                             \
     X(128, 8, 3, 1, 1, 0) X(64, 4, 3, 1, 1, 1) X(64, 4, 3, 2, 2, 1) X(32, 4, 3, 1, 1, 1) X(32, 4, 3, 2, 2, 1)   \
-    X(32, 2, 3, 1, 1, 1) X(32, 2, 3, 2, 2, 1) X(64, 2, 3, 2, 2, 1) X(64, 2, 3, 1, 1, 1)
+    X(32, 2, 3, 1, 1, 1) X(32, 2, 3, 2, 2, 1) X(64, 2, 3, 2, 2, 1) X(64, 2, 3, 1, 1, 1) X(128, 4, 2, 1, 1, 1)           \
+    X(64, 4, 2, 1, 1, 1) X(128, 4, 3, 1, 1, 0)
 
 SkFn pick_sk(int tm, int nwv, int ns, int kg, int kw, int wr, int kind) {
     const int want[6] = {tm, nwv, ns, kg, kw, wr};

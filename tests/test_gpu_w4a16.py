@@ -646,3 +646,21 @@ def test_multi_and_gate_up_many_rows(mcv, oracle, cuda, M, K, Ns):
     act = _host_f32(mcv.mlp_gate_up_silu_w4a16(_to_dev(x), ws[0], wu))
     a_o = oracle.silu_mul(oracle.f2h_rne(refs[0].astype(np.float32)), oracle.f2h_rne(u.astype(np.float32)))
     _check(act, a_o.view(np.float16).astype(np.float32), f"gate_up M={M} K={K} N={Ns[0]}")
+
+
+# The two-stage tiles that share a CU: one to three stages over K (a ring of
+# two), rows and columns past the tile, an output row that is not whole chunks.
+@pytest.mark.parametrize("tm", [128, 64])
+@pytest.mark.parametrize("M,K,N", [(1, 128, 8), (129, 256, 264), (200, 384, 1001)], ids=lambda v: str(v))
+def test_gemm_two_stage_tiles(mcv, oracle, cuda, M, K, N, tm):
+    torch = _torch()
+    x, qweight, qzeros, scales, n8 = _case(tm + M + K + N, M, K, N)
+    w = _dev_weight(mcv, qweight, qzeros, scales)
+    xd = _to_dev(x)
+    out = torch.zeros((M, w.N), dtype=torch.float16, device="cuda")
+    q, s, z = w.ptrs()
+    assert mcv.lib().mcv_w4a16_gemm_sk(xd.data_ptr(), M, K, w.N, q, s, z, 0, out.data_ptr(), tm, 4, 2, 1, 1, 1, 0, 1, None,
+                                       0, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    ref = oracle.w4a16_matmul(x, oracle.unpack_awq(qweight, qzeros), scales)
+    _check(_host_f32(out), ref, f"tm={tm} M={M} K={K} N={N}")
