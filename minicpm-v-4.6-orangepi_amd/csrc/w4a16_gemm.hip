@@ -46,8 +46,8 @@ bool small_output(int64_t M, int64_t N) { return M >= 1 && (M < 8 || M * N < 655
 // cut in whole stages, so they differ by at most one) -- the partial tiles'
 // exchange costs ~1-2 us, which a shorter loop does not pay back.  A
 // tile of four half-slabs takes two k-parts (eight waves, two groups per
-// stage) when its workgroups' group count is even and at least 8 (64-row
-// tiles) or 14 (32-row tiles); the 32 x 64 and 64 x 64 tiles (two
+// stage) when its workgroups' group count is even and at least 8 (32 x 128 at
+// M=130 K=1024 N=3584 6.1 us against 6.8 with one k-part); the 32 x 64 and 64 x 64 tiles (two
 // half-slabs) whenever K/128 is even: two waves per SIMD cover each other's
 // copy issue.  The 64-
 // and 32-row tiles load their weights, zeros and scales straight into
@@ -94,7 +94,7 @@ SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split, bool exact
     constexpr SkConfig kOne[] = {{128, 8, 3, 1}, {64, 4, 3, 1}, {64, 2, 3, 1}, {32, 4, 3, 1}, {32, 2, 3, 1}};
     const int64_t G = K / kGroup;
     auto finish = [&](SkConfig c) {
-        if (G % 2 == 0 && (c.nwv == 2 || (c.nwv == 4 && ((c.tm == 64 && G >= 8) || (c.tm == 32 && G >= 14)))))
+        if (G % 2 == 0 && (c.nwv == 2 || (c.nwv == 4 && G >= 8)))
             c.kg = c.kw = 2;
         c.wr = c.tm != 128;
         return c;
@@ -114,8 +114,11 @@ SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split, bool exact
         double least = 0;
         for (const Cost& k : kCosts) {
             if (exact && k.c.nwv == 8) continue;
-            const int64_t n = ceil_div(w4a16_sk_tiles(M, N, k.c), 256);
-            const double t = n == 1 ? k.one : k.two + static_cast<double>(n - 2) * k.more;
+            const int64_t tk = w4a16_sk_tiles(M, N, k.c), n = ceil_div(tk, 256);
+            // (a round that leaves CUs idle leaves the others more bandwidth and clock:
+            // 128 x 256 at K=3584 37.4 us with 72 tiles, 44.9 with 184, 52.8 with 240)
+            const double t = n == 1 ? k.one * (0.6 + 0.4 * static_cast<double>(tk) / 256)
+                                    : k.two + static_cast<double>(n - 2) * k.more;
             if (least == 0 || t < least) {
                 least = t;
                 best = k.c;
