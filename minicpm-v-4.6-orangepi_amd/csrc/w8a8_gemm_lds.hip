@@ -608,7 +608,7 @@ GemmLFn pick_epi(const ShapeL& s) {
 #define MCV_L(BM_, BN_, NS_, WR_) \
     if (s.bm == BM_ && s.bn == BN_ && s.ns == NS_ && s.wr == WR_) return w8a8_gemm_lds_kernel<BM_, BN_, NS_, EPI, WR_>;
     MCV_L(128, 128, 3, 0) MCV_L(128, 128, 4, 0) MCV_L(64, 128, 4, 0) MCV_L(128, 64, 4, 0) MCV_L(64, 64, 4, 0)
-    MCV_L(64, 64, 3, 0) MCV_L(128, 128, 3, 1) MCV_L(128, 128, 4, 1) MCV_L(64, 128, 4, 1)
+    MCV_L(64, 64, 3, 0) MCV_L(64, 128, 3, 1) MCV_L(128, 128, 3, 1) MCV_L(128, 128, 4, 1) MCV_L(64, 128, 4, 1)
 #undef MCV_L
     return nullptr;
 }
@@ -623,24 +623,34 @@ GemmLFn pick_l(const ShapeL& s, int epi) {
     }
 }
 
-// Largest tiles first; the first shape whose grid covers most of the 256
-// CUs, else the one with the most workgroups.  Measured on MI355X (K=1024,
-// N=3584, 160 rotated weight sets, back to back, two passes of three timed
-// regions): M=1024 128x128 with 3 stages and the weights in registers 7.85-7.90
-// us (through LDS 7.91-7.95, 4 stages 8.26-8.37, 64x128 10.4-11.1, 64x64
-// 11.9-12.2); M=256 64x64 4.72-4.75 us (64x128 6.0-6.15, 128x128 7.4-7.8),
-// and with 3 stages 4.66-4.68 us (2 stages 5.38-5.43; 32x128 with the
-// weights in registers 4.90-4.93 with 3 stages, 5.31-5.34 with 4).
-ShapeL choose_l(int64_t M, int64_t N) {
-    constexpr ShapeL kOrder[] = {{128, 128, 3, 1}, {64, 128, 4, 1}, {64, 64, 3, 0}};
-    ShapeL best = kOrder[0];
-    int64_t best_t = -1;
-    for (const ShapeL& s : kOrder) {
-        const int64_t t = ceil_div(M, s.bm) * ceil_div(N, s.bn);
-        if (t >= 200) return s;
-        if (t > best_t) {
-            best_t = t;
-            best = s;
+// The tile with the least modelled time: a start and output of ~3 us and, per 128
+// of K, what the fullest CU takes with n = 1, 2 or more tiles (two 128 x 128 tiles
+// share a CU).  Measured on MI355X over M = 70..3000 with K=1024 N=3584 and K=3584
+// N=1024 (rotated weights, back to back), us, against the first of 128 x 128, 64 x
+// 128, 64 x 64 to reach 200 workgroups: M=300 K=1024 5.9 -> 5.1 (64 x 128), M=577
+// 8.6 -> 7.0 and M=800 9.1 -> 7.1 (128 x 128 on 140 and 196 CUs), K=3584 M=1500
+// 13.8 -> 11.6 (64 x 128), M=3000 21.3 -> 17.3 (128 x 128 on 192).  The 64-row tiles
+// keep three stages in flight up to K = 1024 (M=256 N=3584 4.7 us, four 4.75; 64 x
+// 128 M=300 5.1 / 5.4) and four on a longer loop (K=3584 M=300 6.7 / 7.8, M=1500
+// 11.6 / 12.1).
+ShapeL choose_l(int64_t M, int64_t K, int64_t N) {
+    struct Cost {
+        ShapeL s;
+        double fixed, one, two, more;
+    };
+    const double G = static_cast<double>(ceil_div(K, 128));
+    const int ns = K < 2048 ? 3 : 4;
+    const Cost costs[] = {{{128, 128, 3, 1}, 3.0, 0.5, 0.95, 0.65},
+                          {{64, 128, ns, 1}, 2.7, 0.31, 0.62, 0.4},
+                          {{64, 64, ns, 0}, 3.1, 0.13, 0.34, 0.27}};
+    ShapeL best = costs[0].s;
+    double least = 0;
+    for (const Cost& c : costs) {
+        const int64_t n = ceil_div(ceil_div(M, c.s.bm) * ceil_div(N, c.s.bn), 256);
+        const double t = c.fixed + G * (n == 1 ? c.one : c.two + static_cast<double>(n - 2) * c.more);
+        if (least == 0 || t < least) {
+            least = t;
+            best = c.s;
         }
     }
     return best;
@@ -648,9 +658,9 @@ ShapeL choose_l(int64_t M, int64_t N) {
 
 }  // namespace
 
-// The kernel launch_w8a8_gemm_lds picks for M x N, as text (report labels).
-std::string w8a8_gemm_lds_name(int64_t M, int64_t N, bool f16) {
-    const ShapeL s = choose_l(M, N);
+// The kernel launch_w8a8_gemm_lds picks for M x K x N, as text (report labels).
+std::string w8a8_gemm_lds_name(int64_t M, int64_t K, int64_t N, bool f16) {
+    const ShapeL s = choose_l(M, K, N);
     char buf[128];
     // EPI as launched with fp32 scales (fp16 ones add 1 and 2)
     std::snprintf(buf, sizeof(buf), "w8a8_gemm_lds_kernel<%d, %d, %d, %d, %d> (%s, %lld workgroups)", s.bm, s.bn,
@@ -696,7 +706,7 @@ int launch_w8a8_gemm_lds_shape(const int8_t* xq, int64_t M, int64_t K, int64_t N
 // As above with the dispatch's tile shape (choose_l).
 int launch_w8a8_gemm_lds(const int8_t* xq, int64_t M, int64_t K, int64_t N, const int8_t* w, void* out, bool f16,
                          const void* xs, int xs16, const void* ws, int ws16, hipStream_t stream) {
-    return launch_w8a8_gemm_lds_shape(xq, M, K, N, w, out, f16, xs, xs16, ws, ws16, choose_l(M, N), stream);
+    return launch_w8a8_gemm_lds_shape(xq, M, K, N, w, out, f16, xs, xs16, ws, ws16, choose_l(M, K, N), stream);
 }
 
 // Any built tile shape (tests and tuning; mcv_w8a8_gemm_lds).

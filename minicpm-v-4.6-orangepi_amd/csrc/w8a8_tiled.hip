@@ -392,7 +392,7 @@ int64_t w8a8_tiled_bytes(int64_t K, int64_t N) {
 
 int launch_w8a8_gemm_lds(const int8_t* xq, int64_t M, int64_t K, int64_t N, const int8_t* w, void* out, bool f16,
                          const void* xs, int xs16, const void* ws, int ws16, hipStream_t stream);
-std::string w8a8_gemm_lds_name(int64_t M, int64_t N, bool f16);
+std::string w8a8_gemm_lds_name(int64_t M, int64_t K, int64_t N, bool f16);
 bool w8a8_uses_rows(int64_t M, int64_t K, int64_t N);
 std::string w8a8_rows_name(int64_t M, int64_t K, int64_t N, bool f16);
 int launch_w8a8_rows(const int8_t* xq, int64_t M, int64_t K, int64_t N, const int8_t* w, void* out, bool f16,
@@ -408,7 +408,7 @@ bool w8a8_uses_gemv(int64_t M, int64_t K) {
 // The kernel launch_w8a8_tiled runs for M x K x N, as text (report labels).
 std::string w8a8_tiled_name(int64_t M, int64_t K, int64_t N, bool f16) {
     if (w8a8_uses_rows(M, K, N)) return w8a8_rows_name(M, K, N, f16);
-    if (!w8a8_uses_gemv(M, K)) return w8a8_gemm_lds_name(M, N, f16);
+    if (!w8a8_uses_gemv(M, K)) return w8a8_gemm_lds_name(M, K, N, f16);
     const int64_t nslab = ceil_div(N, kSlab), KB = ceil_div(K, 128) * 4;
     const bool narrow = nslab < 128;
     const int nw = narrow && KB <= 64 ? 8 : 16, halves = narrow ? 1 : 2, u = narrow && KB <= 64 ? 4 : 2;

@@ -561,3 +561,17 @@ def test_few_rows_bit_exact(mcv, oracle, cuda, M, K, N):
     assert (acc.cpu().numpy() == ref).all()
     assert torch.equal(mcv.matmul_w8a8(xd, sd, w), mcv.w8a8_dequant(acc, sd, w.w_scale_f32))
     assert torch.equal(mcv.matmul_w8a8(xd, sd.half(), w, use_f32_scale=False), mcv.w8a8_dequant(acc, sd.half(), w.w_scale))
+
+
+@pytest.mark.parametrize("M,K,N", [(65, 128, 136), (130, 1040, 1003), (300, 384, 260)], ids=lambda v: str(v))
+def test_w8a8_gemm_three_stage_tiles(mcv, oracle, cuda, M, K, N):
+    """The 64 x 128 tile with three stages: one stage, a partial one, edges."""
+    torch = _torch()
+    rng = np.random.default_rng(M + K + N)
+    xq = rng.integers(-128, 128, (M, K), dtype=np.int8)
+    wq = rng.integers(-127, 128, (K, N), dtype=np.int8)
+    xd, wd = torch.from_numpy(xq).cuda(), torch.from_numpy(mcv.pack_w8a8_tiled(wq)).cuda()
+    acc = torch.empty((M, N), dtype=torch.int32, device="cuda")
+    assert mcv.lib().mcv_w8a8_gemm_lds(xd.data_ptr(), 0, mcv.MCV_F32, M, K, N, wd.data_ptr(), 0, mcv.MCV_F32,
+                                       acc.data_ptr(), 0, 64, 128, 3, 1, torch.cuda.current_stream().cuda_stream) == 0
+    assert (acc.cpu().numpy() == oracle.gemm_i32(xq, wq)).all()
