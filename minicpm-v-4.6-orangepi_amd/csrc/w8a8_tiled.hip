@@ -6,9 +6,9 @@
 //
 // The tiled layout stores every 32-column x 32-k block of the weight as one
 // contiguous 1 KiB line in the operand order of v_mfma_i32_32x32x32_i8 (lane
-// l: column l%32, k-half l/32, 16 bytes).  The GEMM over it (M > 4) stages
-// both operands in LDS (w8a8_gemm_lds.hip); this file holds the layout's
-// GEMV and the dispatch.
+// l: column l%32, k-half l/32, 16 bytes).  The GEMM over it stages both
+// operands in LDS (w8a8_gemm_lds.hip) and the few-row kernels split K over waves
+// (w8a8_rows.hip); this file holds the layout's GEMV and the dispatch.
 //
 // GEMV (M <= 2, where the few-row kernels of w8a8_rows.hip do not take over, and
 // the fused gate + up to M = 4): one workgroup per slab, waves splitting K, v_dot4
@@ -428,15 +428,17 @@ int launch_w8a8_tiled(const int8_t* xq, int64_t M, int64_t K, int64_t N, const i
     if (nslab * KB * 2 * kW8Block >= (int64_t(1) << 32) || M * K >= (int64_t(1) << 32))
         return fail(MCV_ERR_SHAPE, "w8a8 tiled: weight or activation exceeds 4 GiB");
     if (w8a8_uses_rows(M, K, N)) return launch_w8a8_rows(xq, M, K, N, w, out, f16, xs, xs16, ws, ws16, stream);
-    // The GEMV up to M = 4, but only up to M = 2 past K = 2048, where its
-    // serial k-blocks per wave cost more than the GEMM's fixed start
-    // (MI355X, graph-replayed, us: K=3584 N=1024 GEMV M=1/2/4 4.8/6.3/8.4,
-    // GEMM M=5 6.6; K=1024 N=3584 GEMV M=4 3.8, GEMM M=5 4.0).
+    // What the few-row kernels leave of M <= 4 is one row up to K = 2048 or of a
+    // wide output, two rows of a wide one, and weights past their 2 GiB; of the
+    // last the GEMV takes M = 3 and 4 up to K = 2048 only, where its serial
+    // k-blocks per wave cost less than the GEMM's fixed start (MI355X,
+    // graph-replayed, us: K=3584 N=1024 GEMV M=4 8.4, GEMM M=5 6.6; K=1024 N=3584
+    // 3.8, 4.0).
     if (w8a8_uses_gemv(M, K)) {
         return f16 ? launch_w8a8_gemv<true, false>(xq, M, K, N, w, nullptr, out, xs, xs16, ws, nullptr, ws16, stream)
                    : launch_w8a8_gemv<false, false>(xq, M, K, N, w, nullptr, out, xs, xs16, ws, nullptr, ws16, stream);
     }
-    // M > 4: the LDS-staged GEMM (w8a8_gemm_lds.hip)
+    // the rest: the LDS-staged GEMM (w8a8_gemm_lds.hip)
     return launch_w8a8_gemm_lds(xq, M, K, N, w, out, f16, xs, xs16, ws, ws16, stream);
 }
 
