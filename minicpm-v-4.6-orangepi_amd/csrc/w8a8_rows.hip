@@ -76,7 +76,9 @@ __global__ __launch_bounds__(1024) void w8a8_rows_kernel(Rows8Args a) {
                                              static_cast<uint32_t>(rows < 16 * MB ? rows : 16 * MB) * a.K);
     const __amdgpu_buffer_rsrc_t wr = rsrc_8(a.w, static_cast<uint32_t>(a.nslab) * a.KB * 2 * kLine8);
     // x loads: rows 8 t + lane / 8 of a 16-row block, 128 bytes a row; k past K
-    // meets zero weights, rows past M are not used
+    // meets zero weights, rows past M are not used.  The whole offset is the
+    // vector one: where K is not whole groups of 128 the last row's last chunks
+    // lie past x, and the scalar offset is not part of the range check.
     const uint32_t xoff = static_cast<uint32_t>(lane >> 3) * a.K + 16u * (lane & 7);
     uint8_t* const mine = lds + wave * R;
     uint32_t woff[CB];
@@ -111,7 +113,7 @@ __global__ __launch_bounds__(1024) void w8a8_rows_kernel(Rows8Args a) {
 #pragma unroll
                 for (int t = 0; t < 2; ++t)
                     xv[u][b][t] = __builtin_bit_cast(
-                        int4_t, __builtin_amdgcn_raw_buffer_load_b128(xr, (xoff + (16 * b + 8 * t) * a.K) | dead, gc * 128, 0));
+                        int4_t, __builtin_amdgcn_raw_buffer_load_b128(xr, (xoff + (16 * b + 8 * t) * a.K + gc * 128) | dead, 0, 0));
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -187,7 +189,7 @@ __global__ __launch_bounds__(512) void w8a8_rows_wide_kernel(Rows8Args a) {
     for (int t = wave; t < G * MB * 2; t += NW) {         // eight rows of one group
         const int g = t / (2 * MB), m = 8 * (t % (2 * MB)) + (lane >> 3);
         const int4_t v = __builtin_bit_cast(
-            int4_t, __builtin_amdgcn_raw_buffer_load_b128(xr, static_cast<uint32_t>(m) * a.K + 16u * (lane & 7), g * 128, 0));
+            int4_t, __builtin_amdgcn_raw_buffer_load_b128(xr, static_cast<uint32_t>(m) * a.K + 16u * (lane & 7) + g * 128, 0, 0));
         *reinterpret_cast<int4_t*>(lds + (g * MB + (m >> 4)) * 2048 + x8_at(m & 15, lane & 7)) = v;
     }
     __syncthreads();
