@@ -39,7 +39,8 @@ namespace {
 // each); other rows of up to 256 * 16 elements are held element by element,
 // longer ones reloaded (NC = 0).  MI355X, K=3584, 2-byte loads and 1-byte stores
 // against chunks: M=1 3.1 / 2.3 us, M=40 3.4 / 2.6, M=3000 10.0 / 9.0 (a wave per
-// row instead of four: 9.9).
+// row instead of four 9.9; two rows a workgroup, their loads out together, 8.7
+// where one took 7.7); act_quant has the figures since.
 template <int NC, bool VEC>
 __global__ __launch_bounds__(256) void w8a8_quant_act_kernel(const uint16_t* __restrict__ x, int K,
                                                              int8_t* __restrict__ xq, float* __restrict__ s32,
