@@ -114,7 +114,7 @@ def build_cpp_tests(jobs: int | None = None) -> list[Path]:
 
     def one(src: Path) -> Path:
         exe = bindir / src.stem
-        _run(["g++", *CXX_FLAGS, f"-I{oracle}", str(src), "-o", str(exe), f"-L{LIB}", "-lminicpmv_ops", "-lmcv_quant",
+        _run(["g++", *CXX_FLAGS, f"-I{oracle}", f"-I{CSRC}", str(src), "-o", str(exe), f"-L{LIB}", "-lminicpmv_ops", "-lmcv_quant",
               f"-L{oracle / 'build'}", "-lmcv_oracle", "-L/opt/rocm/lib", "-lamdhip64",
               "-Wl,-rpath,$ORIGIN/../../../minicpm-v-4.6-orangepi_amd/lib", "-Wl,-rpath,$ORIGIN/../../../oracle/build",
               "-Wl,-rpath,/opt/rocm/lib"])

@@ -26,6 +26,22 @@ struct W4Parts {
     int count;
 };
 
+// The wide kernel's loads of a group's scales (fp16 [G][Npad]) and zero words
+// (u32 [G][Npad / 8]): lane l < 16 cb takes column n0 + l of the unit, by a
+// vector offset and a scalar base.  The buffer range check covers the vector
+// offset alone, so the base plus the last taking lane's offset has to lie in
+// the buffer, and a lane past the unit's columns gets an offset the check
+// refuses: in the last unit of the last group it would read past the tensors.
+constexpr uint32_t kLoadNothing = 0x80000000u;
+__host__ __device__ constexpr uint32_t wide_scale_offset(int lane, int cb) {
+    return lane < 16 * cb ? static_cast<uint32_t>(lane) * 2u : kLoadNothing;
+}
+__host__ __device__ constexpr uint32_t wide_zero_offset(int lane, int cb) {
+    return lane < 16 * cb ? static_cast<uint32_t>(lane >> 3) * 4u : kLoadNothing;
+}
+__host__ __device__ constexpr int wide_scale_base(int g, int Npad, int n0) { return (g * Npad + n0) * 2; }
+__host__ __device__ constexpr int wide_zero_base(int g, int Npad, int n0) { return (g * (Npad >> 3) + n0 / 8) * 4; }
+
 // True where the few-row kernels are the faster ones for M rows over `nslab`
 // slabs of `parts` weights.
 bool w4a16_rows_pays(int64_t M, int64_t K, int64_t nslab, int parts);

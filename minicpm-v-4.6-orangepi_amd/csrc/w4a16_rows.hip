@@ -251,8 +251,9 @@ __global__ __launch_bounds__(1024) void w4a16_gemv_kernel_rows(const uint16_t* _
 // (1 KiB per group, word and 16 rows); each wave then walks whole slabs on its
 // own, all of K, with the next kWideDepth groups' weights in flight, and
 // stores its 64 columns straight from the accumulators.  A group's scales and
-// zero words come in as one load each for the slab's 64 columns and reach the
-// lanes of each 16-column block through ds_bpermute.  MI355X, K=1024, us, split
+// zero words come in as one load each for the unit's columns (the lanes past
+// them load nothing) and reach the lanes of each 16-column block through
+// ds_bpermute.  MI355X, K=1024, us, split
 // kernel / this one with 32 columns a unit, two groups in flight, 8 waves: M=6
 // V=31012 6.6 / 8.8, 62024 11.2 / 10.2, 124047 19.6 / 15.4, 248094 35.3 / 27.1
 // (64 columns 28.6; four groups in flight 29.3; 4 waves 29.2; 16 waves of 64
@@ -275,6 +276,7 @@ __global__ __launch_bounds__(T) void w4a16_rows_wide_kernel(const uint16_t* __re
     uint32_t woff[CB];
 #pragma unroll
     for (int c = 0; c < CB; ++c) woff[c] = static_cast<uint32_t>(j * kSlab + 16 * c + (lane & 15)) * 16u;
+    const uint32_t soff = wide_scale_offset(lane, CB), zoff = wide_zero_offset(lane, CB);
     uint4 w[D][CB];
     uint32_t s[D], z[D];
     auto load_w = [&](int slot, int unit, int g) {
@@ -286,8 +288,8 @@ __global__ __launch_bounds__(T) void w4a16_rows_wide_kernel(const uint16_t* __re
         for (int c = 0; c < CB; ++c)
             w[slot][c] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
                                                        qr, woff[c] | dead, (slab * C + gc * 4) * 1024 + in * 16, 2));
-        s[slot] = __builtin_amdgcn_raw_buffer_load_b16(sr, (lane * 2u) | dead, (gc * Npad + n0) * 2, 0);
-        z[slot] = __builtin_amdgcn_raw_buffer_load_b32(zr, ((lane >> 3) * 4u) | dead, (gc * (Npad >> 3) + n0 / 8) * 4, 0);
+        s[slot] = __builtin_amdgcn_raw_buffer_load_b16(sr, soff | dead, wide_scale_base(gc, Npad, n0), 0);
+        z[slot] = __builtin_amdgcn_raw_buffer_load_b32(zr, zoff | dead, wide_zero_base(gc, Npad, n0), 0);
     };
     int unit = static_cast<int>(blockIdx.x) * NW + wave;
     const int step = static_cast<int>(gridDim.x) * NW;

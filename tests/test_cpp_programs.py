@@ -99,3 +99,7 @@ def test_cpp_lm_head_from_embedding(tmp_path):
 @pytest.mark.parametrize("mode", [None, "all"])
 def test_cpp_decode_dispatch(mode):
     run("test_decode_dispatch", "dispatch", env={} if mode is None else {"MINICPM_W8A8_DECODE": mode})
+
+
+def test_rows_wide_load_offsets():
+    assert run("test_rows_offsets").strip().endswith("ok")
