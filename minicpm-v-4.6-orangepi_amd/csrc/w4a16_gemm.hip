@@ -24,10 +24,7 @@ int gemv_ksplit(int64_t G, int64_t blocks);
 
 // The few-row kernels aside (w4a16_rows_pays comes first): the GEMV streams the
 // weights once per row and still beats the MFMA GEMM, whose tile count is M/TM
-// * N/TN, until the output reaches about 64K elements; with more than 32 rows
-// only on a short K or a grid of one workgroup per CU (MI355X, rotated weights:
-// M=48 N=1024 K=1024 4.67 us against 4.85; M=40 N=1024 K=3584 12.9 against 7.2,
-// K=2048 8.4 against 6.5).
+// * N/TN, until the output reaches about 64K elements.
 bool small_output(int64_t M, int64_t N) { return M >= 1 && (M < 8 || M * N < 65536); }
 
 // The GEMM's configuration for M x K x N.  First the largest tile whose grid
@@ -137,22 +134,55 @@ SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split, bool exact
     return finish(c);
 }
 
-bool w4a16_prefers_gemv(int64_t M, int64_t K, int64_t N) {
-    return small_output(M, N) && (M <= 32 || K <= 1024 || M * ceil_div(N, kSlab) <= 256);
+bool w4a16_parts_prefer_gemv(int64_t M, int64_t K, int64_t nslab, bool silu) {
+    // The GEMV's grid at which the GEMM, a row tile or two of few workgroups and
+    // without a K split, catches up: the shorter K, the larger; with an odd group
+    // count, which leaves the GEMM one k-part, half as much again.  MI355X, us,
+    // GEMV / GEMM: N=1024 + 1024 M=32 K=128 3.0 / 3.9; N=512 M=33 K=1152 4.4 / 7.0,
+    // K=3072 7.8 / 9.2; gate + up N=512 M=64 K=256 3.8 / 4.5, M=33 K=3584 13.4 / 10.6.  Gate + up of up to 32 rows never runs the GEMM, so
+    // that its bits stay two GEMV calls'.
+    if (M < 8 || (silu && M <= 32)) return true;
+    const int64_t limit = silu ? 192 + 131072 / K : 512 + 196608 / K;
+    return M * nslab <= ((K / kGroup) % 2 != 0 && K > 1024 ? limit + limit / 2 : limit);
 }
 
 namespace {
 
+// One weight, the few-row kernels aside.  Past 32 rows and K = 1024 the GEMV's
+// grid has to stay near two workgroups per CU (one where the GEMM splits K); where
+// an odd group count leaves the GEMM one k-part, any small output up to K = 1408
+// and three workgroups per CU without a split.  MI355X, us, GEMV / GEMM, mean of
+// weights cold and in cache: K=1152 N=512 M=64 4.5 / 6.9; K=1536 N=512 M=64 4.9 / 6.3,
+// N=1000 M=40 6.1 / 6.7, K=1280 M=48 5.7 / 6.1, M=64 6.6 / 6.1; K=2048 N=1000 M=40 8.4 /
+// 7.3 split, 7.5 unsplit; K=3584 12.4 / 7.9, 10.4; K=3968 N=512 M=33 9.4 / 8.3, 15.9.
+bool prefers_gemv(int64_t M, int64_t K, int64_t N, bool can_split) {
+    if (!small_output(M, N)) return false;
+    if (M <= 32 || K <= 1024) return true;
+    const int64_t grid = M * ceil_div(N, kSlab);
+    if ((K / kGroup) % 2 != 0) {
+        if (K <= 1408) return true;
+        if (!can_split) return grid <= 768;
+    }
+    return grid <= (K <= 1536 ? 640 : can_split && K > 2304 ? 256 : 512);
+}
+
+// The few-row kernels by speed: ahead of the GEMV and, where that does not take
+// the call, of the GEMM.
+bool prefers_rows(int64_t M, int64_t K, int64_t N) {
+    const int64_t nslab = ceil_div(N, kSlab);
+    return w4a16_rows_pays(M, K, nslab, 1) && (small_output(M, N) || !w4a16_rows_trail_gemm(M, K, nslab));
+}
+
 // The GEMV or (through launch_w4a16_gemv) the few-row kernels take this call.
 // The few-row kernels and the GEMM need an aligned x and 32-bit offsets; a small
 // output without them runs the GEMV, which needs neither.
-bool takes_gemv(const void* x, int64_t M, int64_t K, int64_t N) {
-    if (w4a16_prefers_gemv(M, K, N)) return true;
+bool takes_gemv(const void* x, int64_t M, int64_t K, int64_t N, bool can_split) {
     if (x == nullptr || M < 2 || K <= 0 || K % kGroup != 0 || N <= 0 || N > (int64_t(1) << 30)) return small_output(M, N);
+    if (prefers_gemv(M, K, N, can_split)) return true;
     W4Parts parts{};
     parts.count = 1;
     parts.p[0].Npad = static_cast<int>(ceil_div(N, kSlab) * kSlab);
-    if (w4a16_rows_pays(M, K, ceil_div(N, kSlab), 1) && w4a16_rows_ok(x, M, K, parts)) return true;
+    if (prefers_rows(M, K, N) && w4a16_rows_ok(x, M, K, parts)) return true;
     return small_output(M, N) && (reinterpret_cast<uintptr_t>(x) % 16 != 0 || !w4a16_sk_fits(M, K, parts));
 }
 
@@ -198,9 +228,7 @@ int mcv_w4a16_gemm_mfma(const void* x, int64_t M, int64_t K, int64_t N, const vo
 }
 
 int64_t mcv_w4a16_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N) {
-    if (M < 1 || K <= 0 || N <= 0 || K % kGroup != 0 || w4a16_prefers_gemv(M, K, N) ||
-        w4a16_rows_pays(M, K, ceil_div(N, kSlab), 1))
-        return 0;
+    if (M < 1 || K <= 0 || N <= 0 || K % kGroup != 0 || prefers_gemv(M, K, N, true) || prefers_rows(M, K, N)) return 0;
     return w4a16_sk_workspace_bytes(M, N, choose_gemm(M, K, N, true));
 }
 
@@ -209,7 +237,7 @@ int64_t mcv_w4a16_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N) {
 int mcv_w4a16_gemm_ws(const void* x, int64_t M, int64_t K, int64_t N, const void* qw, const void* scales,
                       const void* zeros, int zero_bias, void* out, void* workspace, int64_t workspace_bytes,
                       mcv_stream_t stream) {
-    if (takes_gemv(x, M, K, N))
+    if (takes_gemv(x, M, K, N, workspace != nullptr))
         return launch_w4a16_gemv(x, M, K, N, qw, scales, zeros, zero_bias, out, static_cast<hipStream_t>(stream));
     return launch_w4a16_gemm_mfma(x, M, K, N, qw, scales, zeros, zero_bias, out, static_cast<hipStream_t>(stream),
                                   workspace, workspace_bytes);
@@ -219,7 +247,7 @@ int mcv_w4a16_gemm_ws(const void* x, int64_t M, int64_t K, int64_t N, const void
 // goes to the MFMA kernel, which reuses each dequantised operand across rows.
 int mcv_w4a16_gemm(const void* x, int64_t M, int64_t K, int64_t N, const void* qw, const void* scales,
                    const void* zeros, int zero_bias, void* out, mcv_stream_t stream) {
-    if (takes_gemv(x, M, K, N))
+    if (takes_gemv(x, M, K, N, false))
         return launch_w4a16_gemv(x, M, K, N, qw, scales, zeros, zero_bias, out, static_cast<hipStream_t>(stream));
     return launch_w4a16_gemm_mfma(x, M, K, N, qw, scales, zeros, zero_bias, out, static_cast<hipStream_t>(stream),
                                   nullptr, 0);
@@ -229,9 +257,9 @@ const char* mcv_w4a16_gemm_kernel_name(int64_t M, int64_t K, int64_t N, int with
     char buf[160];
     if (M < 1 || K <= 0 || N <= 0 || K % kGroup != 0) {
         g_kernel_name = "none (bad shape)";
-    } else if (w4a16_rows_pays(M, K, ceil_div(N, kSlab), 1)) {
+    } else if (prefers_rows(M, K, N)) {
         g_kernel_name = w4a16_rows_name(M, K, ceil_div(N, kSlab));
-    } else if (w4a16_prefers_gemv(M, K, N)) {
+    } else if (prefers_gemv(M, K, N, with_workspace != 0)) {
         std::snprintf(buf, sizeof(buf), "w4a16_gemv_kernel<%d, 1, 0> (grid %lld x %lld)",
                       gemv_ksplit(K / kGroup, ceil_div(N, kSlab) * M), (long long)ceil_div(N, kSlab), (long long)M);
         g_kernel_name = buf;

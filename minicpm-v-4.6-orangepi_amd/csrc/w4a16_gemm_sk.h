@@ -51,6 +51,8 @@ bool w4a16_sk_fits(int64_t M, int64_t K, const W4Parts& parts);
 // The configuration the dispatch (w4a16_gemm.hip) takes for M x K x N; `exact`:
 // for launch_w4a16_gemm_sk_parts.
 SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split, bool exact = false);
-bool w4a16_prefers_gemv(int64_t M, int64_t K, int64_t N);
+// True where several weights over one x (`nslab` slabs in all) or, with `silu`,
+// gate and up of `nslab` slabs each, run the GEMV rather than that GEMM.
+bool w4a16_parts_prefer_gemv(int64_t M, int64_t K, int64_t nslab, bool silu);
 
 }  // namespace mcv

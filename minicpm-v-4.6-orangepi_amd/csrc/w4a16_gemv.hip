@@ -851,7 +851,7 @@ int mcv_w4a16_gemv_multi(const void* x, int64_t M, int64_t K, const mcv_w4a16_pa
     // over the concatenated column tiles (both read x in 16-byte pieces)
     const hipStream_t st = static_cast<hipStream_t>(stream);
     if (w4a16_rows_pays(M, K, total, n_parts) && w4a16_rows_ok(x, M, K, gp)) return launch_w4a16_rows(x, M, K, gp, st);
-    if (!w4a16_prefers_gemv(M, K, total * kSlab) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && w4a16_sk_fits(M, K, gp))
+    if (!w4a16_parts_prefer_gemv(M, K, total, false) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && w4a16_sk_fits(M, K, gp))
         return launch_w4a16_gemm_sk_parts(x, M, K, gp, nullptr, choose_gemm(M, K, total * kSlab, false, true), st);
     // The k-split the smallest part would get on its own (the decode shapes
     // with K = 1024 all get 8, so the outputs equal separate launches').
@@ -888,7 +888,7 @@ int mcv_w4a16_gate_up_silu(const void* x, int64_t M, int64_t K, int64_t N, const
     const hipStream_t st = static_cast<hipStream_t>(stream);
     if (w4a16_rows_pays(M, K, nslab, 2) && w4a16_rows_ok(x, M, K, parts))
         return launch_w4a16_rows_silu(x, M, K, parts, act, st);
-    if (!w4a16_prefers_gemv(M, K, 2 * nslab * kSlab) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && w4a16_sk_fits(M, K, parts))
+    if (!w4a16_parts_prefer_gemv(M, K, nslab, true) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && w4a16_sk_fits(M, K, parts))
         return launch_w4a16_gemm_sk_parts(x, M, K, parts, act, choose_gemm(M, K, 2 * nslab * kSlab, false, true), st);
     const GemvCfg cfg = choose_gemv(K / kGroup, nslab * M);
     using Fn = void (*)(const uint16_t*, const uint4*, const uint16_t*, const uint32_t*, uint32_t, const uint4*,

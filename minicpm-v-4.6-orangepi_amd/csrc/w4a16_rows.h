@@ -42,9 +42,13 @@ __host__ __device__ constexpr uint32_t wide_zero_offset(int lane, int cb) {
 __host__ __device__ constexpr int wide_scale_base(int g, int Npad, int n0) { return (g * Npad + n0) * 2; }
 __host__ __device__ constexpr int wide_zero_base(int g, int Npad, int n0) { return (g * (Npad >> 3) + n0 / 8) * 4; }
 
-// True where the few-row kernels are the faster ones for M rows over `nslab`
+// True where the few-row kernels are faster than the GEMV for M rows over `nslab`
 // slabs of `parts` weights.
 bool w4a16_rows_pays(int64_t M, int64_t K, int64_t nslab, int parts);
+
+// True where the GEMM is faster than they are, on an output too large for the
+// GEMV (one weight).
+bool w4a16_rows_trail_gemm(int64_t M, int64_t K, int64_t nslab);
 
 // True where the few-row kernels can run this call: at least 2 rows, x
 // 16-byte aligned, x and every packed weight below 2 GiB (32-bit buffer

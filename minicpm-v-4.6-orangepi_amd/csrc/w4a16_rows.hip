@@ -381,13 +381,14 @@ struct RowsCfg {
 };
 
 // 16-row blocks by M; columns per workgroup: the most (64, 32, 16) that still
-// leave about one workgroup per CU.
+// leave about one workgroup per CU, unless fewer would make more than one
+// (65-95 slabs on 16 columns: two rounds; K=2560 N=4608 M=2 6.5 us, on 32 5.1).
 RowsCfg choose_rows(int64_t M, int64_t K, int64_t cols, int nw) {
     RowsCfg c;
     c.mb = M <= 16 ? 1 : 2;
     c.ks = rows_ks(K / kGroup);
     c.cb = 4;
-    while (c.cb > 1 && (cols / (16 * c.cb) < 192 || c.mb * c.cb * nw > 4)) c.cb /= 2;
+    while (c.cb > 1 && ((cols / (16 * c.cb) < 192 && cols / (8 * c.cb) <= 256) || c.mb * c.cb * nw > 4)) c.cb /= 2;
     return c;
 }
 
@@ -455,17 +456,47 @@ bool w4a16_rows_ok(const void* x, int64_t M, int64_t K, const W4Parts& parts) {
     return cols / 16 <= 0x7fffffff;
 }
 
-// The GEMV's grid of one workgroup per slab and row costs little until it
-// exceeds a workgroup per CU, and its rows need no LDS: at K=1024 M=2 N=1024 it
-// takes 2.9 us against 3.2, N=3584 3.1 / 3.2, K=2048 N=1024 M=16 3.9 / 4.1; past
-// K=2048 its two trips over K lose (K=3584 M=2 5.0 / 4.5).  Past 32 rows the
-// GEMM is ahead but for wide outputs (M=48 K=2048 N=1024 6.5 here, 6.6 there;
-// K=3584 9.1 / 7.0).
+// Against the GEMV, whose grid is one workgroup per slab and row.  That grid
+// costs little until it exceeds a workgroup per CU, and its rows need no LDS; the
+// few-row kernel's time hardly depends on M within a 16-row block.  MI355X, us,
+// GEMV / here, mean of weights cold and in cache (measured over K = 128..8192, N =
+// 64..12288, M = 2..32):
+//   grid > 256: K=3584 N=1000 M=32 9.0 / 6.4; but one or two groups leave neither a K
+//   to split, and the GEMV starts sooner: K=128 N=6144 M=5 2.7 / 3.5, K=256 N=6144 M=8
+//   3.2 / 3.5, M=12 3.6 / 3.5; four: N=2048 M=8 2.9 / 3.1; more than 128 slabs on a
+//   short K, where 64-column units are the narrowest to fit a round: K=1024 N=10240
+//   M=2 4.3 / 5.1, M=5 6.2 / 5.1;
+//   grid <= 256, up to 16 rows: past K = 2048 the GEMV's second trip over K loses
+//   (K=3584 N=1000 M=2 5.3 / 4.8) unless its slabs are many (N=4608 5.6 / 5.9); a
+//   shorter K from 32 slabs and 100 workgroups on unless its groups are four or
+//   eight, one per GEMV wave (K=768 N=3584 M=3 3.8 / 3.5, K=1024 3.4 / 3.7);
+//   17 to 32 rows: K=1024 N=512 M=32 3.3 / 3.9, K=2048 N=256 4.0 / 4.7; but one
+//   narrow weight (up to three slabs): K=1152 N=136 M=20 4.0 / 3.6.  Gate and up
+//   together do not (K=2048 N=136 M=32 5.0 / 5.8).
+// Past 32 rows only wide outputs.
 bool w4a16_rows_pays(int64_t M, int64_t K, int64_t nslab, int parts) {
     if (M < 2 || M > 64) return false;
+    const int64_t G = K / kGroup, grid = M * nslab;
+    if (G <= 2 && M <= 3) return false;
     if (parts == 1 && rows_wide(M, K, nslab)) return true;
     if (M > 32) return false;
-    return M > 16 || K > 2048 || (nslab >= 32 && M * nslab > 100) || M * nslab > 256;
+    if (G == 1) return grid > 4096;
+    if (G == 2) return grid > (parts == 1 ? 960 : 640);
+    if (grid > 256) return (G != 4 || grid > 512) && (M > 16 || nslab <= 128 || grid * K > 500000);
+    if (M > 16) return parts == 1 && nslab < 4;
+    return nslab <= 64 && (K > 2048 || (G != 4 && G != 8 && nslab >= 32 && grid > 100));
+}
+
+// Against the GEMM, for outputs too large for the GEMV.  17 to 32 rows of 32-column
+// units take a second round past 128 slabs, where the GEMM's tiles of 32 x 128 do not
+// (K=3584 N=10240 M=32 15.5 us here / 11.8 GEMM) unless an odd group count leaves it
+// one k-part (K=3968 M=17 14.6 / 18.4); one or two groups leave the waves here
+// nothing to split (K=256 N=6144 M=24 4.4 / 4.0, N=4096 3.5 / 4.1).
+bool w4a16_rows_trail_gemm(int64_t M, int64_t K, int64_t nslab) {
+    if (rows_wide(M, K, nslab)) return false;
+    const int64_t G = K / kGroup;
+    if (G <= 2) return G == 1 || nslab > (M <= 16 ? 128 : 64);
+    return M > 16 && G % 2 == 0 && (nslab > 128 || K > 6144);
 }
 
 int launch_w4a16_rows(const void* x, int64_t M, int64_t K, W4Parts parts, hipStream_t stream) {

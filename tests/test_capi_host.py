@@ -504,3 +504,23 @@ def test_embedding_quantisers(mcv, oracle, V, H, N):
     q, s32, _ = mcv.quantize_w8a8_embedding(bf, N, mcv.SRC_BF16, mcv.W8_KN)
     q_o, s_o, _ = oracle.w8a8_quantize_weight(pad16)
     assert np.array_equal(q, q_o) and np.array_equal(s32.view(np.uint32), s_o.view(np.uint32))
+
+
+@pytest.mark.parametrize("M,K,N,ws,want", [
+    # one or two groups, four, many slabs on a short K, few slabs: the GEMV
+    (5, 128, 6144, 1, "w4a16_gemv_kernel<"), (3, 256, 25608, 1, "w4a16_gemv_kernel<"), (8, 512, 2048, 1, "w4a16_gemv_kernel<"),
+    (2, 1024, 10240, 1, "w4a16_gemv_kernel<"), (2, 1024, 3584, 1, "w4a16_gemv_kernel<"), (2, 3584, 4608, 1, "w4a16_gemv_kernel<"),
+    (32, 1024, 512, 1, "w4a16_gemv_kernel<"), (32, 2048, 256, 1, "w4a16_gemv_kernel<"),
+    # past 32 rows: a grid near two workgroups per CU, more without a split
+    (64, 1152, 512, 1, "w4a16_gemv_kernel<"), (40, 1536, 1000, 1, "w4a16_gemv_kernel<"), (64, 2048, 512, 1, "w4a16_gemv_kernel<"),
+    (33, 3968, 512, 0, "w4a16_gemv_kernel<"), (33, 3968, 512, 1, "w4a16_gemm_sk_kernel<"), (40, 3584, 1024, 1, "w4a16_gemm_sk_kernel<"),
+    # the few-row kernels, 72 slabs in one round; the GEMM past 128 slabs
+    (5, 1024, 3584, 1, "w4a16_gemv_kernel_rows<1, 1, "), (32, 3584, 1024, 1, "w4a16_gemv_kernel_rows<2, 1, "),
+    (20, 1152, 136, 1, "w4a16_gemv_kernel_rows<2, 1, "), (5, 2560, 4608, 1, "w4a16_gemv_kernel_rows<1, 2, "),
+    (32, 3584, 10240, 1, "w4a16_gemm_sk_kernel<"), (17, 3968, 10240, 1, "w4a16_gemv_kernel_rows<2, 2, "),
+    (24, 256, 6144, 1, "w4a16_gemm_sk_kernel<"), (6, 1024, 248094, 1, "w4a16_rows_wide_kernel<")], ids=lambda v: str(v))
+def test_w4a16_few_row_routes(mcv, M, K, N, ws, want):
+    """Which kernel one weight runs at the lines of the dispatch's rules."""
+    assert mcv.lib().mcv_w4a16_gemm_kernel_name(M, K, N, ws).decode().startswith(want)
+    if not want.startswith("w4a16_gemm"):
+        assert mcv.lib().mcv_w4a16_gemm_workspace_bytes(M, K, N) == 0 or ws == 0
