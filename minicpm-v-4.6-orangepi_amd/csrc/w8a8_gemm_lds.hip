@@ -632,7 +632,10 @@ GemmLFn pick_l(const ShapeL& s, int epi) {
 // 13.8 -> 11.6 (64 x 128), M=3000 21.3 -> 17.3 (128 x 128 on 192).  The 64-row tiles
 // keep three stages in flight up to K = 1024 (M=256 N=3584 4.7 us, four 4.75; 64 x
 // 128 M=300 5.1 / 5.4) and four on a longer loop (K=3584 M=300 6.7 / 7.8, M=1500
-// 11.6 / 12.1).
+// 11.6 / 12.1).  The table's start and two-tile figures are fitted over K = 128..8192,
+// N = 64..124000, M = 3..3000: on a loop of one or two stages the smallest tile
+// starts soonest (K=128 N=1024 M=300 64 x 64 3.3 us, 64 x 128 3.9), and two 128 x 128
+// tiles a CU are ahead of three or four of 64 x 128 (K=384 N=2048 M=3000 8.1 / 9.5).
 ShapeL choose_l(int64_t M, int64_t K, int64_t N) {
     struct Cost {
         ShapeL s;
@@ -640,9 +643,9 @@ ShapeL choose_l(int64_t M, int64_t K, int64_t N) {
     };
     const double G = static_cast<double>(ceil_div(K, 128));
     const int ns = K < 2048 ? 3 : 4;
-    const Cost costs[] = {{{128, 128, 3, 1}, 3.0, 0.5, 0.95, 0.65},
-                          {{64, 128, ns, 1}, 2.7, 0.31, 0.62, 0.4},
-                          {{64, 64, ns, 0}, 3.1, 0.13, 0.34, 0.27}};
+    const Cost costs[] = {{{128, 128, 3, 1}, 2.8, 0.5, 0.82, 0.65},
+                          {{64, 128, ns, 1}, 2.7, 0.31, 0.7, 0.4},
+                          {{64, 64, ns, 0}, 2.7, 0.13, 0.34, 0.27}};
     ShapeL best = costs[0].s;
     double least = 0;
     for (const Cost& c : costs) {

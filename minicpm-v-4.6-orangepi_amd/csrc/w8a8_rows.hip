@@ -241,8 +241,8 @@ int rows8_ks(int64_t G) { return static_cast<int>(ceil_div(G, ceil_div(G, 16)));
 
 // Whether and how these kernels run M x K x N.  MI355X, rotated weights, us, the
 // GEMV (M <= 4) or GEMM they replace / here:
-//   one row on a long K (the GEMV's two trips): K=3584 N=1024 M=1 5.0 / 3.9, M=2
-//   6.5 / 3.9; M=2 K=1024 N=3584 3.2 / 3.0 but N=6144 3.4 / 3.5; M=4 N=248094
+//   one row on a long K (the GEMV's two trips) up to 64 slabs: K=3584 N=1024 M=1 5.0 /
+//   3.9, N=4608 5.1 / 5.9; two rows, M=2 6.5 / 3.9; M=2 K=1024 N=3584 3.2 / 3.0 but N=6144 3.4 / 3.5; M=4 N=248094
 //   51.7 / 39.8;
 //   up to 32 rows everywhere: K=1024 N=3584 M=5 5.1 / 3.0, M=32 5.2 / 3.5; K=3584
 //   N=1024 M=32 11.7 / 4.5; N=31012 M=32 11.3 / 8.9;
@@ -250,18 +250,27 @@ int rows8_ks(int64_t G) { return static_cast<int>(ceil_div(G, ceil_div(G, 16)));
 //   11.8 / 4.5, M=256 10.5 / 6.6; K=1024 N=3584 M=64 5.3 / 4.0, but M=256 4.8 / 6.6,
 //   N=1024 M=256 3.8 / 3.9.
 // Blocks grow from 16 rows x 16 columns until the grid fits a workgroup per CU
-// (K=3584 N=1024 M=64: 256 of 16 x 16 4.5, 64 of 32 x 32 6.7).
+// (K=3584 N=1024 M=64: 256 of 16 x 16 4.5, 64 of 32 x 32 6.7).  The waves that split K
+// also write the output, so the larger the block the more groups of 128 it takes
+// to pay, GEMV or GEMM / here, mean of weights cold and in cache: one wave K=128
+// N=3584 M=64 3.4 / 6.0 (32 x 32), N=1024 M=96 3.3 / 4.2 (16 x 32); two K=256 N=4608
+// M=8 3.4 / 3.5, N=3072 M=64 3.5 / 4.8; six K=768 N=2048 M=96 4.1 / 4.5; eight K=1024
+// N=3072 M=48 4.6 / 4.2.  A grid of several workgroups per CU hides more of it, but
+// past K = 2048 the GEMM's wider tiles read x less often (K=512 N=31012 M=32 8.4 /
+// 7.4; K=3584 23.8 / 26.7).
 // The wide kernel: N=248094 M=6 50.2 / 40.6, M=16 55.8 / 44.1, M=32 63.3 / 50.6,
 // M=64 85 / 61; at N=62024 it is level with the split kernel (M=32 15.7 both) and
-// behind the GEMM at M=64 (18.6 / 19.7).
+// behind the GEMM at M=64 (18.6 / 19.7), as it is past 32 rows from K = 1536 on (N=124000
+// M=48 40.5 / 45.8).
 bool pick_rows8(int64_t M, int64_t K, int64_t N, Rows8Cfg& c) {
     const int64_t nslab = ceil_div(N, kSlab), G = ceil_div(K, 128);
     if (M < 1 || M > 512 || nslab * G * 8192 >= (int64_t(1) << 31) || M * K >= (int64_t(1) << 31)) return false;
-    if (M == 1 && !(nslab < 128 && K > 2048)) return false;
+    if (M == 1 && !(nslab <= 64 && K > 2048)) return false;
     if (M == 2 && nslab >= 64) return false;
     const int mb = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
     c.ks = rows8_ks(G);
-    c.wide = M <= 64 && nslab >= (mb == 1 ? 2000 : (mb == 2 ? 900 : 1200)) && G * mb * 2048 <= 160 * 1024;
+    c.wide = M <= 64 && nslab >= (mb == 1 ? 2000 : (mb == 2 ? 900 : 1200)) && G * mb * 2048 <= 160 * 1024 &&
+             (mb < 4 || G < 12);
     c.mb = mb;
     c.cb = 2;
     if (c.wide) return true;
@@ -270,7 +279,10 @@ bool pick_rows8(int64_t M, int64_t K, int64_t N, Rows8Cfg& c) {
     c.mb = c.cb = 1;
     if (grid(1, 1) > 256) c.cb = 2;
     if (grid(1, 2) > 256 && M > 16) c.mb = 2;
-    return true;
+    const int64_t wgs = grid(c.mb, c.cb);
+    if (c.mb == 2) return wgs <= 512 ? G >= 7 : G >= 4 && G <= 16;
+    if (c.cb == 2) return G > 2 || wgs > (G == 2 ? 512 : 900);
+    return G > 1 || M > 4;
 }
 
 template <int MB, int CB, bool F16>

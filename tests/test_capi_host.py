@@ -524,3 +524,15 @@ def test_w4a16_few_row_routes(mcv, M, K, N, ws, want):
     assert mcv.lib().mcv_w4a16_gemm_kernel_name(M, K, N, ws).decode().startswith(want)
     if not want.startswith("w4a16_gemm"):
         assert mcv.lib().mcv_w4a16_gemm_workspace_bytes(M, K, N) == 0 or ws == 0
+
+
+@pytest.mark.parametrize("M,K,N,want", [
+    (64, 128, 3584, "w8a8_gemm_lds_kernel<64, 64, 3"), (300, 128, 1024, "w8a8_gemm_lds_kernel<64, 64, 3"),
+    (64, 256, 3072, "w8a8_gemm_lds_kernel<64, 64, 3"), (96, 768, 2048, "w8a8_gemm_lds_kernel<64, 64, 3"),
+    (8, 256, 4608, "w8a8_gemm_lds_kernel<64, 64, 3"), (3000, 384, 2048, "w8a8_gemm_lds_kernel<128, 128, 3"),
+    (40, 1024, 3584, "w8a8_rows_kernel<2, 2, "), (5, 256, 1024, "w8a8_rows_kernel<1, 1, "), (32, 512, 31012, "w8a8_rows_kernel<2, 2, "),
+    (32, 3584, 31012, "w8a8_gemm_lds_kernel<"), (1, 3584, 1024, "w8a8_rows_kernel<1, 1, "), (1, 5120, 4608, "w8a8_tiled_gemv_kernel<"),
+    (16, 1024, 248094, "w8a8_rows_wide_kernel<1, "), (48, 1536, 124000, "w8a8_gemm_lds_kernel<")], ids=lambda v: str(v))
+def test_w8a8_few_row_routes(mcv, M, K, N, want):
+    """Which kernel a tiled W8A8 matmul runs at the lines of the dispatch's rules."""
+    assert mcv.lib().mcv_w8a8_gemm_kernel_name(M, K, N, mcv.W8_TILED, 1).decode().startswith(want)
