@@ -173,7 +173,10 @@ int mcv_w4a16_gemm(const void* x_dev, int64_t M, int64_t K, int64_t N,
  * unsplit) and be zero-filled once before its first use: its first 4 KiB hold
  * the tiles' arrival counters, which every call leaves zero, so one workspace
  * serves calls of every shape.  Calls that share a workspace must be ordered
- * (one stream). */
+ * (one stream); a workspace that a captured graph uses must outlive the graph,
+ * so one of MCV_W4A16_GEMM_WORKSPACE_MAX bytes, which no shape exceeds, never
+ * has to be replaced. */
+#define MCV_W4A16_GEMM_WORKSPACE_MAX (4096 + 256 * 32 * 64 * 4)
 int mcv_w4a16_gemm_ws(const void* x_dev, int64_t M, int64_t K, int64_t N,
                       const void* qw_dev, const void* scales_dev, const void* zeros_dev,
                       int zero_bias, void* out_dev, void* workspace_dev, int64_t workspace_bytes,
@@ -182,6 +185,11 @@ int mcv_w4a16_gemm_ws(const void* x_dev, int64_t M, int64_t K, int64_t N,
 /* Workspace bytes mcv_w4a16_gemm_ws uses for this shape (0: it does not split
  * K, and any workspace, NULL included, is ignored). */
 int64_t mcv_w4a16_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N);
+
+/* 0 when `stream` is not under graph capture, else a number that tells this
+ * capture from every other (a library that keeps workspaces gives each graph its
+ * own).  Never fails: a stream that cannot be asked is not under capture. */
+int64_t mcv_stream_capture_id(mcv_stream_t stream);
 
 /* The kernel (and configuration) mcv_w4a16_gemm (with_workspace = 0) or
  * mcv_w4a16_gemm_ws (1) launches for M x K x N, as text, for labels in

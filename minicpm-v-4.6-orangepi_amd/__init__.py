@@ -69,6 +69,7 @@ _SIGS = {
     "mcv_w4a16_gemm": (_c_int, [_vp, _c_i64, _c_i64, _c_i64, _vp, _vp, _vp, _c_int, _vp, _vp]),
     "mcv_w4a16_gemm_ws": (_c_int, [_vp, _c_i64, _c_i64, _c_i64, _vp, _vp, _vp, _c_int, _vp, _vp, _c_i64, _vp]),
     "mcv_w4a16_gemm_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
+    "mcv_stream_capture_id": (_c_i64, [_vp]),
     "mcv_w4a16_gemm_kernel_name": (ctypes.c_char_p, [_c_i64, _c_i64, _c_i64, _c_int]),
     "mcv_w8a8_gemm_kernel_name": (ctypes.c_char_p, [_c_i64, _c_i64, _c_i64, _c_int, _c_int]),
     "mcv_w4a16_gemm_sk_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_int, _c_int, _c_int]),
@@ -456,29 +457,63 @@ def _gemm_workspace_bytes(M: int, K: int, N: int) -> int:
     return int(lib().mcv_w4a16_gemm_workspace_bytes(M, K, N))
 
 
-_GEMM_WS: dict = {}
+# MCV_W4A16_GEMM_WORKSPACE_MAX and the bytes of its tile counters.
+GEMM_WORKSPACE_BYTES = 4096 + 256 * 32 * 64 * 4
+_GEMM_COUNTER_BYTES = 4096
+_GEMM_WS: dict = {}            # (device, stream, bytes) -> workspace
+_GEMM_WS_CAPTURE: dict = {}    # the same -> (capture id, workspace of that graph)
 
 
 def gemm_workspace(nbytes: int, device, stream=None):
-    """The K-split workspace of the W4A16 GEMM for calls on one stream: kept
-    per (device, stream), zero-filled when (re)allocated -- its tile counters
-    must start at zero, and every call leaves them zero -- and grown only when
-    a shape needs more, so steady-state calls allocate nothing.  Calls on one
-    stream are ordered, so they may share it; two streams never do."""
+    """The K-split workspace of the W4A16 GEMM for calls on one stream: one per
+    (device, stream), large enough for every shape, zero-filled on that stream
+    -- its tile counters must start at zero, and every call leaves them zero
+    -- and then kept, so later calls allocate nothing.  Calls on one stream are
+    ordered, so they may share it; two streams never do.
+
+    A graph captured on a stream that has one records it, so its replays count
+    as calls on that stream.  On any other stream the graph gets its own, from
+    its memory pool and cleared by one of its kernels, and shares nothing.  (Its
+    own on every stream would cost the clearing kernel's ~1.5 us per replay.)"""
     torch = _torch()
     dev = torch.device(device)
-    key = (dev.index if dev.index is not None else torch.cuda.current_device(), _stream(stream))
+    handle = _stream(stream)
+    key = (dev.index if dev.index is not None else torch.cuda.current_device(), handle,
+           max(nbytes, GEMM_WORKSPACE_BYTES))
     ws = _GEMM_WS.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
-        _GEMM_WS[key] = ws
-    return ws
+    if ws is not None:
+        return ws
+    capture = lib().mcv_stream_capture_id(handle)
+    if capture == 0:
+        return _GEMM_WS.setdefault(key, _workspace_on(key[2], key[2], dev, handle, stream))
+    held = _GEMM_WS_CAPTURE.get(key)
+    if held is None or held[0] != capture:
+        held = (capture, _workspace_on(key[2], _GEMM_COUNTER_BYTES, dev, handle, stream))
+        _GEMM_WS_CAPTURE[key] = held
+    return held[1]
+
+
+def _workspace_on(nbytes: int, zeroed: int, dev, handle: int, stream):
+    """Device bytes allocated, and the first `zeroed` of them cleared, on that stream."""
+    torch = _torch()
+
+    def make():
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        ws[:zeroed].zero_()
+        return ws
+
+    if handle == _stream():
+        return make()
+    if not isinstance(stream, torch.cuda.Stream):
+        stream = torch.cuda.ExternalStream(handle, device=dev) if handle else torch.cuda.default_stream(dev)
+    with torch.cuda.stream(stream):
+        return make()
 
 
 def matmul_w4a16(x, w: W4A16QuantizedWeight, out=None, stream=None):
     """out[M, N] = x[M, K] . dequant(w), any M (ops.h:104-108 generalised).
     Where the MFMA GEMM splits K across workgroups (few rows, long K) it takes
-    the per-stream workspace of gemm_workspace()."""
+    the workspace of gemm_workspace()."""
     torch = _torch()
     if x.dtype != torch.float16 or x.dim() != 2 or x.shape[1] != w.K or not x.is_contiguous():
         raise McvError(f"matmul_w4a16: x must be contiguous fp16 [M, {w.K}]")

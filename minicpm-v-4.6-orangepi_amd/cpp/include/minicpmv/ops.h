@@ -35,14 +35,17 @@ void matmul_w4a16(const Tensor& x, const Tensor& w_int8, const Tensor& scales, T
 // x fp16 [M, K] . dequant(w) -> out fp16 [M, N], any M (GEMV for small M,
 // LDS-dequant fp16 MFMA GEMM otherwise).  Where the GEMM splits K across
 // workgroups it uses a workspace the library keeps per (device, stream) of
-// the calling thread: allocated on the first call that needs it (or more of
-// it), reused after that.
+// the calling thread: allocated once, large enough for every shape, on the
+// first call that needs it.  Under graph capture, where nothing can be
+// allocated, a stream without one runs unsplit; a graph that recorded one is
+// ordered with that stream's calls, as calls on the stream are.
 void matmul_w4a16(const Tensor& x, const W4A16QuantizedWeight& w, Tensor& out, hipStream_t stream);
 
 // The same with a caller-owned workspace (mcv_w4a16_gemm_ws): where the MFMA
 // path splits K across workgroups (few rows, long K) its fp32 partial tiles go
-// there.  `workspace` (Int8) is reallocated only when a shape needs more than
-// it holds; calls that share it must be ordered on one stream.
+// there.  `workspace` (Int8) is allocated when a shape needs more than it
+// holds, at MCV_W4A16_GEMM_WORKSPACE_MAX bytes, so once (and not under capture:
+// the call then runs unsplit); calls that share it must be ordered on one stream.
 void matmul_w4a16(const Tensor& x, const W4A16QuantizedWeight& w, Tensor& out, hipStream_t stream, Tensor& workspace);
 
 // Decode MLP front half in one launch: act [M, I] = silu(x . gate) * (x . up),

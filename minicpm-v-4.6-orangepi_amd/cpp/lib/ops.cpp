@@ -10,6 +10,7 @@
 
 #include <rocblas/rocblas.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <stdexcept>
@@ -30,14 +31,29 @@ void require_slab(const W4A16QuantizedWeight& w, const char* what) {
                                          "than 16 levels); only matmul_w4a16 takes it");
 }
 
-// The workspace of the 4-argument matmul_w4a16: one per (device, stream) of
-// this thread, grown on demand and kept, so calls on one stream reuse it in
-// stream order and calls on two streams never share one.
+// The workspaces of the 4-argument matmul_w4a16: one per (device, stream) of
+// this thread, kept, so calls on one stream reuse it in stream order and calls
+// on two streams never share one.  One that a captured graph recorded stays
+// allocated when the thread ends: the graph may still be replayed.
+struct ImplicitWorkspaces {
+    struct Entry {
+        Tensor workspace;
+        bool captured = false;
+    };
+    std::map<std::pair<int, hipStream_t>, Entry> per_stream;
+    ~ImplicitWorkspaces() {
+        for (auto& [key, e] : per_stream)
+            if (e.captured) new Tensor(std::move(e.workspace));
+    }
+};
+
 Tensor& implicit_gemm_workspace(hipStream_t stream) {
-    thread_local std::map<std::pair<int, hipStream_t>, Tensor> per_stream;
+    thread_local ImplicitWorkspaces held;
     int dev = 0;
     check_hip(hipGetDevice(&dev), "hipGetDevice");
-    return per_stream[{dev, stream}];
+    ImplicitWorkspaces::Entry& e = held.per_stream[{dev, stream}];
+    if (mcv_stream_capture_id(stream) != 0 && e.workspace.data() != nullptr) e.captured = true;
+    return e.workspace;
 }
 
 int scale_dtype(const Tensor& t, const char* what) {
@@ -95,13 +111,18 @@ void matmul_w4a16(const Tensor& x, const W4A16QuantizedWeight& w, Tensor& out, h
     }
     require(w.w_int8.data() && w.scales.data() && w.zeros.data(), "matmul_w4a16 weight is not loaded");
     const int64_t nb = mcv_w4a16_gemm_workspace_bytes(x.shape()[0], w.K, w.N);
-    if (nb > 0 && static_cast<int64_t>(workspace.numel()) < nb) {
-        // the split's tile counters must start at zero (calls leave them zero)
-        workspace = Tensor({nb}, DType::Int8);
-        workspace.zero();
+    if (nb > 0 && static_cast<int64_t>(workspace.numel()) < nb && mcv_stream_capture_id(stream) == 0) {
+        // large enough for every shape, so that a graph that recorded it never sees
+        // it replaced; the split's tile counters must start at zero (calls leave
+        // them zero)
+        workspace = Tensor({std::max<int64_t>(nb, MCV_W4A16_GEMM_WORKSPACE_MAX)}, DType::Int8);
+        workspace.allocate();
+        check_hip(hipMemsetAsync(workspace.data(), 0, workspace.size_bytes(), stream), "hipMemsetAsync");
     }
+    // (memory cannot be allocated under capture: without a workspace the call runs unsplit)
+    const bool split = nb > 0 && static_cast<int64_t>(workspace.numel()) >= nb;
     check_mcv(mcv_w4a16_gemm_ws(x.data(), x.shape()[0], w.K, w.N, w.w_int8.data(), w.scales.data(), w.zeros.data(),
-                                w.zero_bias, out.data(), nb > 0 ? workspace.data() : nullptr, nb, stream),
+                                w.zero_bias, out.data(), split ? workspace.data() : nullptr, split ? nb : 0, stream),
               "matmul_w4a16");
 }
 

@@ -124,6 +124,7 @@ SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split, bool exact
         // the 128 x 128 and three-per-CU shapes are what the table says
         return best.ns == 2 || (best.tm == 128 && best.nwv == 4) ? best : finish(best);
     }
+    static_assert(kSkCounterBytes + 256 * 32 * 64 * 4 == MCV_W4A16_GEMM_WORKSPACE_MAX, "tiles * splits <= 256");
     if (!can_split) return finish(c);
     // the K split: the most ways within 256 workgroups that leave at least 7
     // groups per workgroup on average, cut in whole stages (two groups each
@@ -139,8 +140,9 @@ bool w4a16_parts_prefer_gemv(int64_t M, int64_t K, int64_t nslab, bool silu) {
     // without a K split, catches up: the shorter K, the larger; with an odd group
     // count, which leaves the GEMM one k-part, half as much again.  MI355X, us,
     // GEMV / GEMM: N=1024 + 1024 M=32 K=128 3.0 / 3.9; N=512 M=33 K=1152 4.4 / 7.0,
-    // K=3072 7.8 / 9.2; gate + up N=512 M=64 K=256 3.8 / 4.5, M=33 K=3584 13.4 / 10.6.  Gate + up of up to 32 rows never runs the GEMM, so
-    // that its bits stay two GEMV calls'.
+    // K=3072 7.8 / 9.2; gate + up N=512 M=64 K=256 3.8 / 4.5, M=33 K=3584 13.4 / 10.6.
+    // Gate + up of up to 32 rows never runs the GEMM, so that its bits stay two GEMV
+    // calls'.
     if (M < 8 || (silu && M <= 32)) return true;
     const int64_t limit = silu ? 192 + 131072 / K : 512 + 196608 / K;
     return M * nslab <= ((K / kGroup) % 2 != 0 && K > 1024 ? limit + limit / 2 : limit);
@@ -230,6 +232,17 @@ int mcv_w4a16_gemm_mfma(const void* x, int64_t M, int64_t K, int64_t N, const vo
 int64_t mcv_w4a16_gemm_workspace_bytes(int64_t M, int64_t K, int64_t N) {
     if (M < 1 || K <= 0 || N <= 0 || K % kGroup != 0 || prefers_gemv(M, K, N, true) || prefers_rows(M, K, N)) return 0;
     return w4a16_sk_workspace_bytes(M, N, choose_gemm(M, K, N, true));
+}
+
+int64_t mcv_stream_capture_id(mcv_stream_t stream) {
+    if (stream == nullptr) return 0;                     // the default stream cannot be captured
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream), &status, &id) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return status == hipStreamCaptureStatusNone ? 0 : static_cast<int64_t>(id + 1);
 }
 
 // mcv_w4a16_gemm with a caller-owned workspace, which lets the MFMA path

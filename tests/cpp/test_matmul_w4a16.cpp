@@ -6,12 +6,14 @@
 // (w8 = q - 8 packed as AutoAWQ with zero 8) through the weight overload.
 #include "minicpmv/hip_context.h"
 #include "minicpmv/ops.h"
+#include "mcv_quant.h"
 #include "minicpmv/quantized_weight.h"
 #include "test_common.h"
 
 #include <algorithm>
 #include <cmath>
 #include <random>
+#include <thread>
 
 using namespace minicpmv;
 
@@ -196,6 +198,95 @@ int main() {
                     int(wsp.data() == first));
         if (nb <= 0 || static_cast<int64_t>(wsp.numel()) < nb || worst > 2e-3 || r2 != r3 || wsp.data() != first)
             return 1;
+    }
+
+    // 3b) The workspace of the K split is never replaced: 40 rows (K=3584 N=1024)
+    // first, 128 after.  Both calls captured into one graph give the eager bits,
+    // replayed after larger eager calls; captured on a stream that holds no
+    // workspace yet (nothing can be allocated then) they run unsplit, and the
+    // graph outlives the thread that captured it.
+    {
+        constexpr int KD = 3584, ND = 1024;
+        std::uniform_int_distribution<int> qd(0, 15);
+        std::vector<int32_t> dq(static_cast<size_t>(KD) * ND / 8), dz(static_cast<size_t>(KD / G) * ND / 8, 0x77777777);
+        std::vector<uint16_t> ds(static_cast<size_t>(KD / G) * ND);
+        for (auto& v : dq) {
+            uint32_t word = 0;
+            for (int sl = 0; sl < 8; ++sl) word |= static_cast<uint32_t>(qd(rng)) << (4 * sl);
+            v = static_cast<int32_t>(word);
+        }
+        for (auto& v : ds) v = t::f2h(sd(rng));
+        W4A16QuantizedWeight down = pack_w4a16_awq(dq.data(), dz.data(), ds.data(), KD, ND);
+        std::vector<uint16_t> ha(static_cast<size_t>(128) * KD);
+        for (auto& v : ha) v = t::f2h(xd(rng));
+        Tensor a40({40, KD}, DType::Float16), a128({128, KD}, DType::Float16), o40({40, ND}, DType::Float16),
+            o128({128, ND}, DType::Float16);
+        a40.copy_from_host(ha.data(), static_cast<size_t>(40) * KD * 2);
+        a128.copy_from_host(ha.data(), ha.size() * 2);
+        o40.allocate();
+        o128.allocate();
+        auto host = [&](const Tensor& o) {
+            std::vector<uint16_t> h(o.numel());
+            o.copy_to_host(h.data(), h.size() * 2);
+            return h;
+        };
+        Tensor wsp;
+        matmul_w4a16(a40, down, o40, ctx.stream(), wsp);
+        const void* const first = wsp.data();
+        matmul_w4a16(a128, down, o128, ctx.stream(), wsp);
+        ctx.synchronize();
+        const bool kept = wsp.data() == first && wsp.numel() == MCV_W4A16_GEMM_WORKSPACE_MAX;
+        const std::vector<uint16_t> want40 = host(o40), want128 = host(o128);
+        int bad_replays = 0, cold_ok = 0;
+        auto captures = [&] {
+            for (bool cold : {false, true}) {
+                hipStream_t s = nullptr;
+                check_hip(hipStreamCreate(&s), "hipStreamCreate");
+                if (!cold) {
+                    matmul_w4a16(a40, down, o40, s);           // this thread's workspace for s
+                    check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
+                }
+                hipGraph_t graph = nullptr;
+                hipGraphExec_t exec = nullptr;
+                check_hip(hipStreamBeginCapture(s, hipStreamCaptureModeGlobal), "hipStreamBeginCapture");
+                matmul_w4a16(a40, down, o40, s);
+                matmul_w4a16(a128, down, o128, s);
+                check_hip(hipStreamEndCapture(s, &graph), "hipStreamEndCapture");
+                check_hip(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "hipGraphInstantiate");
+                for (int rep = 0; rep < 3; ++rep) {
+                    check_hip(hipMemset(o40.data(), 0, o40.size_bytes()), "hipMemset");
+                    check_hip(hipMemset(o128.data(), 0, o128.size_bytes()), "hipMemset");
+                    if (!cold) matmul_w4a16(a128, down, o128, s);
+                    check_hip(hipGraphLaunch(exec, s), "hipGraphLaunch");
+                    check_hip(hipStreamSynchronize(s), "hipStreamSynchronize");
+                    if (!cold) {
+                        bad_replays += host(o40) != want40 || host(o128) != want128;
+                        continue;
+                    }
+                    double worst = 0.0;
+                    const std::vector<uint16_t> got = host(o128);
+                    for (size_t i = 0; i < got.size(); ++i) {
+                        const double u = t::h2f(want128[i]), v = t::h2f(got[i]);
+                        worst = std::max(worst, std::fabs(u - v) / (std::fabs(u) + 1e-2));
+                    }
+                    cold_ok += worst <= 2e-3;
+                }
+                check_hip(hipGraphExecDestroy(exec), "hipGraphExecDestroy");
+                check_hip(hipGraphDestroy(graph), "hipGraphDestroy");
+                check_hip(hipStreamDestroy(s), "hipStreamDestroy");
+            }
+        };
+        std::thread([&] {
+            try {
+                captures();
+            } catch (const std::runtime_error& e) {
+                std::printf("%s\n", e.what());
+                bad_replays = -1;
+            }
+        }).join();
+        std::printf("split-K workspace: kept %d, bad replays %d, cold captures unsplit %d of 3\n", int(kept), bad_replays,
+                    cold_ok);
+        if (!kept || bad_replays != 0 || cold_ok != 3) return 1;
     }
 
     // 4) shape validation mirrors the reference's host wrapper
