@@ -43,7 +43,8 @@ __device__ __forceinline__ uint4 rms_chunk(const uint4& x, const uint4& g, float
 // after the sum made two and more.  MI355X, us before / after: M=1 H=1024 2.7 /
 // 2.4, H=3584 5.1 / 3.6, M=1100 H=1024 4.1 / 3.4, M=3000 7.5 / 6.4; with the
 // quantisation M=1 H=1024 3.5 / 3.1, H=2048 4.9 / 3.5.  PER = 0: rows longer than
-// 256 * 32, strided loops.
+// 256 * 32, strided loops, each with only the loads and stores it needs (with the
+// store conditional inside: M=1 H=16384 27.8 us, now 26.3, as before PER).
 template <int PER, bool VEC, bool QUANT>
 __global__ __launch_bounds__(256) void rms_row_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ gamma,
                                                       int H, float eps, uint16_t* __restrict__ normed,
@@ -120,19 +121,23 @@ __global__ __launch_bounds__(256) void rms_row_kernel(const uint16_t* __restrict
         }
     } else {
         const float rstd = row_rstd(xr, H, eps);
-        for (int i = t; i < H; i += blockDim.x) {
-            const uint16_t h = rms_apply(xr[i], rstd, gamma[i]);
-            if constexpr (QUANT) {
+        if constexpr (!QUANT) {
+            for (int i = t; i < H; i += blockDim.x) nr[i] = rms_apply(xr[i], rstd, gamma[i]);
+        } else {
+            auto each = [&](auto&& use) {
+                for (int i = t; i < H; i += blockDim.x) use(i, rms_apply(xr[i], rstd, gamma[i]));
+            };
+            auto largest = [&](uint16_t h) {
                 const float v = fabsf(h2f(h));
                 m = v > m ? v : m;
-            }
-            if (nr) nr[i] = h;
-        }
-        if constexpr (QUANT) {
+            };
+            if (nr) each([&](int i, uint16_t h) { largest(h); nr[i] = h; });
+            else each([&](int, uint16_t h) { largest(h); });
             scale = act_scale(row_absmax(m));
             const float inv = __fdiv_rn(1.0f, scale);
-            // the normed row again: from memory where it was stored (in place, x is gone)
-            for (int i = t; i < H; i += blockDim.x) qr[i] = act_quant(nr ? nr[i] : rms_apply(xr[i], rstd, gamma[i]), inv);
+            // the normed row again, from memory only where x is gone (in place)
+            if (nr == xr) for (int i = t; i < H; i += blockDim.x) qr[i] = act_quant(nr[i], inv);
+            else each([&](int i, uint16_t h) { qr[i] = act_quant(h, inv); });
         }
     }
     if constexpr (QUANT) {
@@ -146,7 +151,9 @@ __global__ __launch_bounds__(256) void rms_row_kernel(const uint16_t* __restrict
 using RmsFn = void (*)(const uint16_t*, const uint16_t*, int, float, uint16_t*, int8_t*, float*, uint16_t*);
 
 // Launches the kernel for M rows of H; VEC needs whole 16-byte chunks: H a
-// multiple of 8 and aligned rows.  (A wave per row, without barriers, was slower
+// multiple of 8 and aligned rows, and more than one element a thread: up to 256
+// it loads x twice where the strided form has everything in one load each
+// (M=50000 H=128 33.3 us in chunks, 24.3 strided; M=8192 H=256 7.8 / 6.3).  (A wave per row, without barriers, was slower
 // below 8192 rows: M=512 H=1024 3.9 us against 3.1, M=2000 H=2048 13.6 / 7.9.)
 template <bool QUANT>
 void launch_rms(const uint16_t* x, const uint16_t* gamma, int64_t M, int64_t H, float eps, uint16_t* normed, int8_t* xq,
@@ -156,7 +163,7 @@ void launch_rms(const uint16_t* x, const uint16_t* gamma, int64_t M, int64_t H, 
     const bool vec = H % 8 == 0 && at % 16 == 0;
     const int h = static_cast<int>(H);
     RmsFn fn = rms_row_kernel<0, false, QUANT>;
-    if (H <= 256) fn = vec ? rms_row_kernel<1, true, QUANT> : rms_row_kernel<1, false, QUANT>;
+    if (H <= 256) fn = rms_row_kernel<1, false, QUANT>;
     else if (H <= 1024) fn = vec ? rms_row_kernel<4, true, QUANT> : rms_row_kernel<4, false, QUANT>;
     else if (H <= 2048) fn = vec ? rms_row_kernel<8, true, QUANT> : rms_row_kernel<8, false, QUANT>;
     else if (H <= 4096) fn = vec ? rms_row_kernel<16, true, QUANT> : rms_row_kernel<16, false, QUANT>;

@@ -161,3 +161,16 @@ def test_argmax_long_rows(mcv, oracle, cuda, M, N):
         x[3] = 0xFC00                                                    # all -inf: 0
     got = mcv.argmax_last_dim(_f16_dev(x)).cpu().numpy()
     assert got.tolist() == [oracle.argmax_f16(x[m]) for m in range(M)]
+
+
+# Onto its own input, the row reread for the quantisation only after it is stored.
+@pytest.mark.parametrize("M,H", [(3, 128), (2, 256), (5, 1024), (3, 8200), (2, 16384)])
+def test_rms_norm_w8a8_quantize_in_place(mcv, cuda, M, H):
+    torch = _torch()
+    rng = np.random.default_rng(M + H)
+    xd, gd = _f16_dev(f16_normal(rng, (M, H), 1.5)), _f16_dev(f16_normal(rng, (H,), 1.0))
+    want, wq, ws, _ = mcv.rms_norm_w8a8_quantize(xd, gd, 1e-6)
+    _, nq, ns, _ = mcv.rms_norm_w8a8_quantize(xd, gd, 1e-6, want_normed=False)
+    got, gq, gs, _ = mcv.rms_norm_w8a8_quantize(xd, gd, 1e-6, normed=xd)
+    assert got.data_ptr() == xd.data_ptr() and torch.equal(got, want)
+    assert torch.equal(gq, wq) and torch.equal(gs, ws) and torch.equal(nq, wq) and torch.equal(ns, ws)
