@@ -30,9 +30,10 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restric
 // Greedy argmax of fp16 rows, first maximum, with argmax_key16's order: NaN and
 // -inf never win, subnormals and -0 count as +0.
 //
-// One workgroup of 1024 threads per row, read in 16-byte chunks of eight values,
-// four in flight per lane (eight: rows of 31012 4.9 us against 4.1, longer ones the
-// same).
+// One workgroup of 1024 threads per row, read in 16-byte chunks of eight values, U
+// = 4 in flight per lane (eight: rows of 31012 4.9 us against 4.1, longer ones the
+// same).  U = 1: rows that leave a lane one chunk, which stays in registers for the
+// lookup below (one row of 8192: per value 3.7 us, U = 4 4.1, U = 1 3.4).
 // What bounds it is the VALU work per value, so a chunk is compared as a whole:
 // packed 16-bit integer steps map a value to a signed order (rank16) in which
 // every value that cannot win sits below kRankNone, a packed maximum folds the
@@ -70,6 +71,7 @@ __device__ __forceinline__ int rank_max8(const uint4& q) {
 }
 
 constexpr int kArgThreads = 1024;
+template <int U>
 __global__ __launch_bounds__(kArgThreads) void argmax_kernel(const uint16_t* __restrict__ x, int64_t N,
                                                              int64_t* __restrict__ idx) {
     const uint16_t* xr = x + static_cast<size_t>(blockIdx.x) * N;
@@ -80,7 +82,7 @@ __global__ __launch_bounds__(kArgThreads) void argmax_kernel(const uint16_t* __r
     const int64_t nv = (N - head) / 8;
     int br = kRankNone;                          // best rank so far and its first chunk
     int64_t bc = 0;
-    constexpr int U = 4;
+    uint4 bq = make_uint4(0, 0, 0, 0);           // U = 1: the lane's only chunk
     for (int64_t j0 = tid; j0 < nv; j0 += int64_t(kArgThreads) * U) {
         uint4 q[U];
 #pragma unroll
@@ -95,6 +97,10 @@ __global__ __launch_bounds__(kArgThreads) void argmax_kernel(const uint16_t* __r
             br = take ? r : br;
             bc = take ? j0 + int64_t(u) * kArgThreads : bc;
         }
+        if constexpr (U == 1) {
+            bq = q[0];
+            break;
+        }
     }
     unsigned long long best = 0ull;
     auto visit = [&](int64_t i) {
@@ -102,8 +108,8 @@ __global__ __launch_bounds__(kArgThreads) void argmax_kernel(const uint16_t* __r
         best = k > best ? k : best;
     };
     if (br > kRankNone) {
-        const uint4 q = v[bc];
-        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+        if constexpr (U != 1) bq = v[bc];
+        const uint32_t w[4] = {bq.x, bq.y, bq.z, bq.w};
         int first = 7;
 #pragma unroll
         for (int e = 7; e >= 0; --e) first = rank_flush(rank16(w[e / 2])[e & 1]) == br ? e : first;
@@ -150,8 +156,8 @@ int mcv_argmax_f16(const void* x, int64_t M, int64_t N, int64_t* idx, mcv_stream
         return fail(MCV_ERR_SHAPE, "argmax: bad shape M=%lld N=%lld", (long long)M, (long long)N);
     int rc = require_device();
     if (rc != MCV_OK) return rc;
-    hipLaunchKernelGGL(argmax_kernel, dim3(static_cast<unsigned>(M)), dim3(kArgThreads), 0, static_cast<hipStream_t>(stream),
-                       static_cast<const uint16_t*>(x), N, idx);
+    hipLaunchKernelGGL((N <= 8 * kArgThreads ? argmax_kernel<1> : argmax_kernel<4>), dim3(static_cast<unsigned>(M)),
+                       dim3(kArgThreads), 0, static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(x), N, idx);
     return check_launch("argmax_kernel");
 }
 

@@ -174,3 +174,18 @@ def test_rms_norm_w8a8_quantize_in_place(mcv, cuda, M, H):
     got, gq, gs, _ = mcv.rms_norm_w8a8_quantize(xd, gd, 1e-6, normed=xd)
     assert got.data_ptr() == xd.data_ptr() and torch.equal(got, want)
     assert torch.equal(gq, wq) and torch.equal(gs, ws) and torch.equal(nq, wq) and torch.equal(ns, ws)
+
+
+# Rows about the length that leaves every lane one chunk, from aligned and
+# unaligned starts: the maximum in the first and last chunk, a tie, every bit
+# pattern.
+@pytest.mark.parametrize("N", [8, 64, 8184, 8191, 8192, 8193, 8200, 8207])
+def test_argmax_one_chunk_rows(mcv, oracle, cuda, N):
+    rng = np.random.default_rng(N)
+    x = f16_normal(rng, (5, N), 1.0)
+    x[0, 0] = x[1, N - 1] = 0x7C00
+    x[2, [N // 2, N - 1]] = 0x7B00
+    x[3] = rng.integers(0, 65536, N, dtype=np.uint16)
+    x[4] = 0xFE00
+    got = mcv.argmax_last_dim(_f16_dev(x)).cpu().numpy()
+    assert got.tolist() == [oracle.argmax_f16(x[m]) for m in range(5)]
