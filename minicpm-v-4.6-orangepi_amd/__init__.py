@@ -347,7 +347,10 @@ def _stream(stream=None) -> int:
     if stream is not None:
         return int(stream.cuda_stream)
     torch = _torch()
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)      # not a public name
+    if raw is None:
+        return int(torch.cuda.current_stream().cuda_stream)
+    return raw(torch.cuda.current_device())
 
 
 def _dev(t) -> int:

@@ -536,3 +536,13 @@ def test_w4a16_few_row_routes(mcv, M, K, N, ws, want):
 def test_w8a8_few_row_routes(mcv, M, K, N, want):
     """Which kernel a tiled W8A8 matmul runs at the lines of the dispatch's rules."""
     assert mcv.lib().mcv_w8a8_gemm_kernel_name(M, K, N, mcv.W8_TILED, 1).decode().startswith(want)
+
+
+def test_stream_handle_without_the_raw_query(mcv, monkeypatch):
+    """A torch without its private raw-stream query: the public call."""
+    import torch
+    from types import SimpleNamespace
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: SimpleNamespace(cuda_stream=4711))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    assert mcv._stream() == 4711 and mcv._stream(SimpleNamespace(cuda_stream=5)) == 5
