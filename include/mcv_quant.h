@@ -197,6 +197,11 @@ int64_t mcv_stream_capture_id(mcv_stream_t stream);
  * counterpart. */
 const char* mcv_w4a16_gemm_kernel_name(int64_t M, int64_t K, int64_t N, int with_workspace);
 
+/* The same for mcv_w4a16_gemv_multi over `n_parts` weights of `nslab` 64-column
+ * slabs in all (gate_up = 0), or mcv_w4a16_gate_up_silu (1, n_parts 2, `nslab`
+ * those of gate).  No reference counterpart. */
+const char* mcv_w4a16_parts_kernel_name(int64_t M, int64_t K, int64_t nslab, int n_parts, int gate_up);
+
 /* The half-slab GEMM with an explicit configuration (what mcv_w4a16_gemm_ws
  * picks by shape; exposed so every configuration can be tested and timed):
  * tile tm x 32 * waves (tm in {32, 64, 128}, waves in {2, 4, 8}), `stages`

@@ -71,6 +71,7 @@ _SIGS = {
     "mcv_w4a16_gemm_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "mcv_stream_capture_id": (_c_i64, [_vp]),
     "mcv_w4a16_gemm_kernel_name": (ctypes.c_char_p, [_c_i64, _c_i64, _c_i64, _c_int]),
+    "mcv_w4a16_parts_kernel_name": (ctypes.c_char_p, [_c_i64, _c_i64, _c_i64, _c_int, _c_int]),
     "mcv_w8a8_gemm_kernel_name": (ctypes.c_char_p, [_c_i64, _c_i64, _c_i64, _c_int, _c_int]),
     "mcv_w4a16_gemm_sk_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_int, _c_int, _c_int]),
     "mcv_w4a16_gemm_sk": (_c_int, [_vp, _c_i64, _c_i64, _c_i64, _vp, _vp, _vp, _c_int, _vp, _c_int, _c_int, _c_int,

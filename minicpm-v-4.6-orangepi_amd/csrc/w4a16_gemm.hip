@@ -271,17 +271,28 @@ const char* mcv_w4a16_gemm_kernel_name(int64_t M, int64_t K, int64_t N, int with
     if (M < 1 || K <= 0 || N <= 0 || K % kGroup != 0) {
         g_kernel_name = "none (bad shape)";
     } else if (prefers_rows(M, K, N)) {
-        g_kernel_name = w4a16_rows_name(M, K, ceil_div(N, kSlab));
+        g_kernel_name = w4a16_rows_name(M, K, ceil_div(N, kSlab), 1, false);
     } else if (prefers_gemv(M, K, N, with_workspace != 0)) {
         std::snprintf(buf, sizeof(buf), "w4a16_gemv_kernel<%d, 1, 0> (grid %lld x %lld)",
                       gemv_ksplit(K / kGroup, ceil_div(N, kSlab) * M), (long long)ceil_div(N, kSlab), (long long)M);
         g_kernel_name = buf;
     } else {
         const SkConfig c = choose_gemm(M, K, N, with_workspace != 0);
-        std::snprintf(buf, sizeof(buf), "w4a16_gemm_sk_kernel<%d, %d, %d, %d, %d, %d> (K split %d ways, %lld workgroups)%s",
-                      c.tm, c.nwv, c.ns, c.kg, c.kw, c.wr, c.splits, (long long)(w4a16_sk_tiles(M, N, c) * c.splits),
-                      w4a16_sk_config_valid(M, K, N, c) ? "" : " NOT BUILT");
-        g_kernel_name = buf;
+        g_kernel_name = w4a16_sk_name(c, 0, w4a16_sk_tiles(M, N, c) * c.splits);
+        if (!w4a16_sk_config_valid(M, K, N, c)) g_kernel_name += " NOT VALID";
+    }
+    return g_kernel_name.c_str();
+}
+
+const char* mcv_w4a16_parts_kernel_name(int64_t M, int64_t K, int64_t nslab, int n_parts, int gate_up) {
+    if (M < 1 || K <= 0 || K % kGroup != 0 || nslab <= 0 || n_parts < 1 || n_parts > kMaxParts || (gate_up && n_parts != 2)) {
+        g_kernel_name = "none (bad shape)";
+    } else if (w4a16_rows_pays(M, K, nslab, n_parts)) {
+        g_kernel_name = w4a16_rows_name(M, K, nslab, n_parts, gate_up != 0);
+    } else if (w4a16_parts_prefer_gemv(M, K, nslab, gate_up != 0)) {
+        g_kernel_name = gate_up ? "w4a16_gate_up_silu_kernel" : "w4a16_gemv_multi_kernel";
+    } else {
+        g_kernel_name = w4a16_sk_name(choose_gemm(M, K, (gate_up ? 2 : 1) * nslab * kSlab, false, true), gate_up ? 2 : 1, 0);
     }
     return g_kernel_name.c_str();
 }

@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <string>
 
 #include "w4a16_rows.h"
 
@@ -46,6 +47,10 @@ int launch_w4a16_gemm_sk(const void* x, int64_t M, int64_t K, int64_t N, const v
 // `act` part 0 the gate and part 1 the up weight of silu(x . gate) * (x . up).
 int launch_w4a16_gemm_sk_parts(const void* x, int64_t M, int64_t K, const W4Parts& parts, void* act, const SkConfig& c,
                                hipStream_t stream);
+// The kernel's configuration as text: its first six template arguments, KIND (0
+// one weight, 1 several, 2 gate and up) and whether its weight operands are the
+// exact q - z or the rounded (q - z) s.
+std::string w4a16_sk_name(const SkConfig& c, int kind, int64_t workgroups);
 // True where the GEMM's 32-bit buffer offsets cover this call.
 bool w4a16_sk_fits(int64_t M, int64_t K, const W4Parts& parts);
 // The configuration the dispatch (w4a16_gemm.hip) takes for M x K x N; `exact`:

@@ -723,11 +723,11 @@ using SkFn = void (*)(const uint16_t*, W4Parts, uint16_t*, int, int, int, int, i
 // M=2048 19.95 / 19.03, and 64 x 64 M=256 7.03 / 6.81.
 constexpr int one_exact(int tm, int nwv, int, int, int, int) { return tm == 32 || (tm == 64 && nwv == 4) ? 1 : 0; }
 
-// what the dispatch picks (choose_gemm), for several weights
+// what the dispatch picks (choose_gemm with exact operands), for several weights
 #define MCV_SK_PARTS_SHAPES(X)                                                                             \
-    X(128, 8, 3, 1, 1, 0) X(64, 4, 3, 1, 1, 1) X(64, 4, 3, 2, 2, 1) X(32, 4, 3, 1, 1, 1) X(32, 4, 3, 2, 2, 1)   \
-    X(32, 2, 3, 1, 1, 1) X(32, 2, 3, 2, 2, 1) X(64, 2, 3, 2, 2, 1) X(64, 2, 3, 1, 1, 1) X(128, 4, 2, 1, 1, 1)           \
-    X(64, 4, 2, 1, 1, 1) X(128, 4, 3, 1, 1, 0)
+    X(64, 4, 3, 1, 1, 1) X(64, 4, 3, 2, 2, 1) X(32, 4, 3, 1, 1, 1) X(32, 4, 3, 2, 2, 1) X(32, 2, 3, 1, 1, 1)   \
+    X(32, 2, 3, 2, 2, 1) X(64, 2, 3, 2, 2, 1) X(64, 2, 3, 1, 1, 1) X(128, 4, 2, 1, 1, 1) X(64, 4, 2, 1, 1, 1)   \
+    X(128, 4, 3, 1, 1, 0)
 
 SkFn pick_sk(int tm, int nwv, int ns, int kg, int kw, int wr, int kind) {
     const int want[6] = {tm, nwv, ns, kg, kw, wr};
@@ -762,6 +762,17 @@ bool w4a16_sk_config_valid(int64_t M, int64_t K, int64_t N, const SkConfig& c) {
     return pick_sk(c.tm, c.nwv, c.ns, c.kg, c.kw, c.wr, kOne) != nullptr && c.splits >= 1 && c.splits <= 64 && K % kGroup == 0 &&
            (K / kGroup) % c.kg == 0 && c.splits <= K / kGroup / c.kg &&
            (c.splits == 1 || w4a16_sk_tiles(M, N, c) <= kSkMaxSplitTiles);
+}
+
+std::string w4a16_sk_name(const SkConfig& c, int kind, int64_t workgroups) {
+    char buf[176];
+    const int ex = kind == kOne ? one_exact(c.tm, c.nwv, c.ns, c.kg, c.kw, c.wr) : 1;
+    char grid[48] = "";
+    if (workgroups > 0) std::snprintf(grid, sizeof(grid), ", %lld workgroups", static_cast<long long>(workgroups));
+    std::snprintf(buf, sizeof(buf), "w4a16_gemm_sk_kernel<%d, %d, %d, %d, %d, %d> (K split %d ways%s, KIND %d, %s operands)%s",
+                  c.tm, c.nwv, c.ns, c.kg, c.kw, c.wr, c.splits, grid, kind, ex ? "exact" : "rounded",
+                  pick_sk(c.tm, c.nwv, c.ns, c.kg, c.kw, c.wr, kind) != nullptr ? "" : " NOT BUILT");
+    return buf;
 }
 
 bool w4a16_sk_fits(int64_t M, int64_t K, const W4Parts& parts) {

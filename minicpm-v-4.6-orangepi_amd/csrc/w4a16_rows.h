@@ -62,7 +62,8 @@ int launch_w4a16_rows(const void* x, int64_t M, int64_t K, W4Parts parts, hipStr
 // the sums are launch_w4a16_rows' and round to fp16 before silu_mul_f16.
 int launch_w4a16_rows_silu(const void* x, int64_t M, int64_t K, W4Parts parts, void* act, hipStream_t stream);
 
-// The kernel's configuration for M x K over `cols` padded columns, as text.
-const char* w4a16_rows_name(int64_t M, int64_t K, int64_t nslab);
+// The kernel's configuration for M x K over `nslab` slabs of `parts` weights
+// (`silu`: of gate and of up), as text.
+const char* w4a16_rows_name(int64_t M, int64_t K, int64_t nslab, int parts, bool silu);
 
 }  // namespace mcv

@@ -23,8 +23,8 @@
 //
 // Workgroup: KS waves split the groups (wave w takes w, w + KS, ...), each
 // over 16 CB columns and 16 MB rows; the fp32 partial sums meet in LDS and are
-// added in wave order.  KS is the same for every launch with the same K and
-// MB, so a weight's output does not depend on what else the launch computes.
+// added in wave order.  KS is the same for every launch with the same K, so
+// here a weight's output does not depend on what else the launch computes.
 //
 // x passes through LDS: loaded row by row (16 lanes read 256 contiguous bytes)
 // and read back in operand order, because the operand's own order touches 32
@@ -248,12 +248,13 @@ __global__ __launch_bounds__(1024) void w4a16_gemv_kernel_rows(const uint16_t* _
 
 // ---- wide outputs (the lm_head over a few rows): HBM bound, so no split and
 // no exchange.  x is staged once per workgroup in LDS in MFMA operand order
-// (1 KiB per group, word and 16 rows); each wave then walks whole slabs on its
-// own, all of K, with the next kWideDepth groups' weights in flight, and
-// stores its 64 columns straight from the accumulators.  A group's scales and
-// zero words come in as one load each for the unit's columns (the lanes past
-// them load nothing) and reach the lanes of each 16-column block through
-// ds_bpermute.  MI355X, K=1024, us, split
+// (1 KiB per group, word and 16 rows); each wave then takes one unit of 16 CB
+// columns over all of K, with the next D groups' weights in flight, and stores
+// its columns straight from the accumulators.  Its groups add up one after
+// another, the split kernel's per wave and then over the waves, so the last
+// bits of the two differ.  A group's scales and zero words come in as one load
+// each for the unit's columns (the lanes past them load nothing) and reach the
+// lanes of each 16-column block through ds_bpermute.  MI355X, K=1024, us, split
 // kernel / this one with 32 columns a unit, two groups in flight, 8 waves: M=6
 // V=31012 6.6 / 8.8, 62024 11.2 / 10.2, 124047 19.6 / 15.4, 248094 35.3 / 27.1
 // (64 columns 28.6; four groups in flight 29.3; 4 waves 29.2; 16 waves of 64
@@ -291,8 +292,7 @@ __global__ __launch_bounds__(T) void w4a16_rows_wide_kernel(const uint16_t* __re
         s[slot] = __builtin_amdgcn_raw_buffer_load_b16(sr, soff | dead, wide_scale_base(gc, Npad, n0), 0);
         z[slot] = __builtin_amdgcn_raw_buffer_load_b32(zr, zoff | dead, wide_zero_base(gc, Npad, n0), 0);
     };
-    int unit = static_cast<int>(blockIdx.x) * NW + wave;
-    const int step = static_cast<int>(gridDim.x) * NW;
+    const int unit = static_cast<int>(blockIdx.x) * NW + wave;
     if (unit < units) {
 #pragma unroll
         for (int d = 0; d < D; ++d) load_w(d, unit, d);
@@ -304,6 +304,7 @@ __global__ __launch_bounds__(T) void w4a16_rows_wide_kernel(const uint16_t* __re
         *reinterpret_cast<int4_t*>(xl + g * MB * 4096 + x_at(m >> 4, m & 15, lane & 15)) = v;
     }
     __syncthreads();
+    if (unit >= units) return;
 
     uint32_t vmagic;
     asm("v_mov_b32 %0, 0x64006400" : "=v"(vmagic));
@@ -311,67 +312,61 @@ __global__ __launch_bounds__(T) void w4a16_rows_wide_kernel(const uint16_t* __re
     const uint32_t mhi = __builtin_amdgcn_readfirstlane(0x00F000F0u);
     const half2_t sixteenth = as_h2(0x2C002C00u);        // half2(1/16)
 
-    for (; unit < units; unit += step) {
-        float4_t acc[MB][CB];
+    float4_t acc[MB][CB];
 #pragma unroll
-        for (int b = 0; b < MB; ++b)
+    for (int b = 0; b < MB; ++b)
 #pragma unroll
-            for (int c = 0; c < CB; ++c) acc[b][c] = float4_t{0.f, 0.f, 0.f, 0.f};
-        for (int g0 = 0; g0 < G; g0 += D) {
+        for (int c = 0; c < CB; ++c) acc[b][c] = float4_t{0.f, 0.f, 0.f, 0.f};
+    for (int g0 = 0; g0 < G; g0 += D) {
 #pragma unroll
-            for (int u = 0; u < D; ++u) {
-                const int g = g0 + u;                    // past G: zero weights and scales, x of the last group
-                const int gx = g < G ? g : G - 1;
-                // scale (low half) and zero (high half) of this lane's column of the slab
-                const uint32_t sz = (s[u] & 0xffffu) | ((((z[u] >> ((lane & 7) * 4)) & 15u) + P.zero_bias) << 16);
-                half8_t xv[MB][4];
+        for (int u = 0; u < D; ++u) {
+            const int g = g0 + u;                    // past G: zero weights and scales, x of the last group
+            const int gx = g < G ? g : G - 1;
+            // scale (low half) and zero (high half) of this lane's column of the slab
+            const uint32_t sz = (s[u] & 0xffffu) | ((((z[u] >> ((lane & 7) * 4)) & 15u) + P.zero_bias) << 16);
+            half8_t xv[MB][4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int b = 0; b < MB; ++b)
-                        xv[b][i] = *reinterpret_cast<const half8_t*>(xl + gx * MB * 4096 + x_at(b, lane & 15, 4 * j + i));
+                for (int b = 0; b < MB; ++b)
+                    xv[b][i] = *reinterpret_cast<const half8_t*>(xl + gx * MB * 4096 + x_at(b, lane & 15, 4 * j + i));
 #pragma unroll
-                for (int c = 0; c < CB; ++c) {
-                    const uint32_t v = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(
-                        (16 * c + (lane & 15)) * 4, static_cast<int>(sz)));
-                    const uint32_t zq = v >> 16;
-                    const half2_t zlo = as_h2((0x6400u + zq) * 0x10001u);            // 1024 + z
-                    const half2_t zhi = as_h2((0xD400u + (zq << 4)) * 0x10001u);     // -(64 + z)
-                    const uint32_t words[4] = {w[u][c].x, w[u][c].y, w[u][c].z, w[u][c].w};
-                    float4_t ga[MB];
+            for (int c = 0; c < CB; ++c) {
+                const uint32_t v = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(
+                    (16 * c + (lane & 15)) * 4, static_cast<int>(sz)));
+                const uint32_t zq = v >> 16;
+                const half2_t zlo = as_h2((0x6400u + zq) * 0x10001u);            // 1024 + z
+                const half2_t zhi = as_h2((0xD400u + (zq << 4)) * 0x10001u);     // -(64 + z)
+                const uint32_t words[4] = {w[u][c].x, w[u][c].y, w[u][c].z, w[u][c].w};
+                float4_t ga[MB];
 #pragma unroll
-                    for (int b = 0; b < MB; ++b) ga[b] = float4_t{0.f, 0.f, 0.f, 0.f};
+                for (int b = 0; b < MB; ++b) ga[b] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const half8_t wv = widen_exact(words[i], zlo, zhi, mlo, mhi, vmagic, sixteenth);
+                for (int i = 0; i < 4; ++i) {
+                    const half8_t wv = widen_exact(words[i], zlo, zhi, mlo, mhi, vmagic, sixteenth);
 #pragma unroll
-                        for (int b = 0; b < MB; ++b) ga[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[b][i], wv, ga[b], 0, 0, 0);
-                    }
-                    const float sc = h2f(static_cast<uint16_t>(v));
-#pragma unroll
-                    for (int b = 0; b < MB; ++b)
-#pragma unroll
-                        for (int r = 0; r < 4; ++r) acc[b][c][r] = fmaf(ga[b][r], sc, acc[b][c][r]);
+                    for (int b = 0; b < MB; ++b) ga[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xv[b][i], wv, ga[b], 0, 0, 0);
                 }
-                load_w(u, unit, g + D);
+                const float sc = h2f(static_cast<uint16_t>(v));
+#pragma unroll
+                for (int b = 0; b < MB; ++b)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[b][c][r] = fmaf(ga[b][r], sc, acc[b][c][r]);
             }
+            load_w(u, unit, g + D);
         }
-        if (unit + step < units) {
-#pragma unroll
-            for (int d = 0; d < D; ++d) load_w(d, unit + step, d);
-        }
-#pragma unroll
-        for (int b = 0; b < MB; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int m = 16 * b + 4 * j + r;
-#pragma unroll
-                for (int c = 0; c < CB; ++c) {
-                    const int n = (unit * CB + c) * 16 + (lane & 15);
-                    if (m < M && n < P.N) P.out[static_cast<size_t>(m) * P.N + n] = f2h(acc[b][c][r]);
-                }
-            }
     }
+#pragma unroll
+    for (int b = 0; b < MB; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = 16 * b + 4 * j + r;
+#pragma unroll
+            for (int c = 0; c < CB; ++c) {
+                const int n = (unit * CB + c) * 16 + (lane & 15);
+                if (m < M && n < P.N) P.out[static_cast<size_t>(m) * P.N + n] = f2h(acc[b][c][r]);
+            }
+        }
 }
 
 struct RowsCfg {
@@ -513,15 +508,16 @@ int launch_w4a16_rows_silu(const void* x, int64_t M, int64_t K, W4Parts parts, v
     return launch_any<true>(x, M, K, parts, act, stream);
 }
 
-const char* w4a16_rows_name(int64_t M, int64_t K, int64_t nslab) {
+const char* w4a16_rows_name(int64_t M, int64_t K, int64_t nslab, int parts, bool silu) {
     char buf[128];
-    if (rows_wide(M, K, nslab)) {
+    if (parts == 1 && rows_wide(M, K, nslab)) {
         std::snprintf(buf, sizeof(buf), "w4a16_rows_wide_kernel<%d, %d, 2, 512>", M <= 16 ? 1 : (M <= 32 ? 2 : 4),
                       M > 32 && nslab >= 1536 ? 4 : 2);
     } else {
-        const RowsCfg c = choose_rows(M, K, nslab * kSlab, 1);
-        std::snprintf(buf, sizeof(buf), "w4a16_gemv_kernel_rows<%d, %d, %d, false> (%lld workgroups of %d waves)", c.mb, c.cb,
-                      K / kGroup > c.ks && c.mb * c.cb <= 2 ? 2 : 1, (long long)(nslab * 4 / c.cb), c.ks);
+        const RowsCfg c = choose_rows(M, K, nslab * kSlab, silu ? 2 : 1);
+        std::snprintf(buf, sizeof(buf), "w4a16_gemv_kernel_rows<%d, %d, %d, %s> (%lld workgroups of %d waves)", c.mb, c.cb,
+                      K / kGroup > c.ks && c.mb * c.cb <= 2 ? 2 : 1, silu ? "true" : "false", (long long)(nslab * 4 / c.cb),
+                      c.ks);
     }
     g_rows_name = buf;
     return g_rows_name.c_str();
