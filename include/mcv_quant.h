@@ -243,11 +243,11 @@ int mcv_w4a16_gemm_mfma(const void* x_dev, int64_t M, int64_t K, int64_t N,
 
 /* Decode MLP front half in one launch: act[M][N] = silu(x . Wgate) * (x . Wup)
  * with gate and up rounded to fp16 first, as two mcv_w4a16_gemv calls followed
- * by mcv_silu_mul produce it (bit-identical up to 32 rows; beyond, the same
- * exact q - z and fp32 sums in the GEMM's order).  Both weights are K x N
- * slab-64.  Replaces the gate matmul + up matmul + silu_mul sequence of the
+ * by mcv_silu_mul produce it: bit-identical for up to 16 rows and N <= 51136,
+ * and for 17 to 32 rows and 192 < N <= 25536; elsewhere the same exact q - z and
+ * fp32 sums, added in another order.  Both weights are K x N slab-64.  Replaces the gate matmul + up matmul + silu_mul sequence of the
  * decoder layers' MLP (src/csrc/lib/decoder_layer.cpp:1029-1046, silu_mul
- * src/csrc/lib/ops.cpp:437-456).  Any M. */
+ * src/csrc/lib/ops.cpp:437-456).  1 <= M <= 65535. */
 int mcv_w4a16_gate_up_silu(const void* x_dev, int64_t M, int64_t K, int64_t N,
                            const void* qw_gate_dev, const void* scales_gate_dev, const void* zeros_gate_dev,
                            int zero_bias_gate, const void* qw_up_dev, const void* scales_up_dev,
@@ -312,7 +312,7 @@ typedef struct mcv_w4a16_part {
  * (:1108-1110), which the reference dispatches one matmul_decode_dispatch at a
  * time.  Each part's output equals mcv_w4a16_gemv on that weight when both run
  * the same kernel and split K the same way (M = 1: every K = 1024 decode shape);
- * at larger M the fp32 sums may be added in another order.  Any M. */
+ * at larger M the fp32 sums may be added in another order.  1 <= M <= 65535. */
 int mcv_w4a16_gemv_multi(const void* x_dev, int64_t M, int64_t K, const mcv_w4a16_part* parts, int n_parts,
                          mcv_stream_t stream);
 

@@ -573,9 +573,10 @@ def matmul_w4a16_mfma(x, w, out=None, stream=None):
 
 
 def mlp_gate_up_silu_w4a16(x, w_gate: W4A16QuantizedWeight, w_up: W4A16QuantizedWeight, out=None, stream=None):
-    """act[M, N] = silu(x . gate) * (x . up), one launch, any M; up to 32 rows
+    """act[M, N] = silu(x . gate) * (x . up), one launch, up to 65535 rows;
     bit-identical to two matmul_w4a16_gemv calls and silu_mul
-    (decoder_layer.cpp:1029-1046)."""
+    (decoder_layer.cpp:1029-1046) for up to 16 rows and N <= 51136 and for 17 to
+    32 rows and 192 < N <= 25536, elsewhere equal but for the order of the sums."""
     torch = _torch()
     if x.dtype != torch.float16 or x.dim() != 2 or x.shape[1] != w_gate.K or not x.is_contiguous():
         raise McvError(f"mlp_gate_up_silu: x must be contiguous fp16 [M, {w_gate.K}]")

@@ -49,8 +49,9 @@ void matmul_w4a16(const Tensor& x, const W4A16QuantizedWeight& w, Tensor& out, h
 void matmul_w4a16(const Tensor& x, const W4A16QuantizedWeight& w, Tensor& out, hipStream_t stream, Tensor& workspace);
 
 // Decode MLP front half in one launch: act [M, I] = silu(x . gate) * (x . up),
-// gate/up rounded to fp16 first -- bit-identical to two matmul_w4a16 calls and
-// silu_mul (the reference's sequence, decoder_layer.cpp:1029-1046).
+// gate/up rounded to fp16 first, as two matmul_w4a16 calls and silu_mul do (the
+// reference's sequence, decoder_layer.cpp:1029-1046): at M = 1 bit for bit, at
+// larger M the order of the sums may differ (mcv_w4a16_gate_up_silu).
 void mlp_gate_up_silu_w4a16(const Tensor& x, const W4A16QuantizedWeight& gate, const W4A16QuantizedWeight& up,
                             Tensor& act, hipStream_t stream);
 

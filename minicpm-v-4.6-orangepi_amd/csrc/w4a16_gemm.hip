@@ -88,7 +88,7 @@ SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split, bool exact
         {{32, 4, 3, 1}, 0.42, 0.65, 0.55},                     // 32 x 128
         {{32, 2, 3, 1}, 0.3, 0.47, 0.27},                      // 32 x 64
     };
-    constexpr SkConfig kOne[] = {{128, 8, 3, 1}, {64, 4, 3, 1}, {64, 2, 3, 1}, {32, 4, 3, 1}, {32, 2, 3, 1}};
+    constexpr SkConfig kRound[] = {{128, 8, 3, 1}, {64, 4, 3, 1}, {64, 2, 3, 1}, {32, 4, 3, 1}, {32, 2, 3, 1}};
     const int64_t G = K / kGroup;
     auto finish = [&](SkConfig c) {
         if (G % 2 == 0 && (c.nwv == 2 || (c.nwv == 4 && G >= 8)))
@@ -99,7 +99,7 @@ SkConfig choose_gemm(int64_t M, int64_t K, int64_t N, bool can_split, bool exact
     // one tile per workgroup and one workgroup per CU where a tile fits that
     // (200-256 tiles); exact operands (several weights) leave the 128 x 256 tile
     // out, whose registers they fill (gate + up M=1100 21.4 us and here 21.4-21.9, qkv + z 30.1 and 26.3)
-    for (const SkConfig& c : kOne) {
+    for (const SkConfig& c : kRound) {
         if (exact && c.nwv == 8) continue;
         const int64_t t = w4a16_sk_tiles(M, N, c);
         if (t >= 200 && t <= 256) return finish(c);
@@ -172,7 +172,7 @@ bool prefers_gemv(int64_t M, int64_t K, int64_t N, bool can_split) {
 // the call, of the GEMM.
 bool prefers_rows(int64_t M, int64_t K, int64_t N) {
     const int64_t nslab = ceil_div(N, kSlab);
-    return w4a16_rows_pays(M, K, nslab, 1) && (small_output(M, N) || !w4a16_rows_trail_gemm(M, K, nslab));
+    return w4a16_rows_pays(M, K, nslab, kOne) && (small_output(M, N) || !w4a16_rows_trail_gemm(M, K, nslab));
 }
 
 // The GEMV or (through launch_w4a16_gemv) the few-row kernels take this call.
@@ -271,28 +271,30 @@ const char* mcv_w4a16_gemm_kernel_name(int64_t M, int64_t K, int64_t N, int with
     if (M < 1 || K <= 0 || N <= 0 || K % kGroup != 0) {
         g_kernel_name = "none (bad shape)";
     } else if (prefers_rows(M, K, N)) {
-        g_kernel_name = w4a16_rows_name(M, K, ceil_div(N, kSlab), 1, false);
+        g_kernel_name = w4a16_rows_name(M, K, ceil_div(N, kSlab), kOne);
     } else if (prefers_gemv(M, K, N, with_workspace != 0)) {
         std::snprintf(buf, sizeof(buf), "w4a16_gemv_kernel<%d, 1, 0> (grid %lld x %lld)",
                       gemv_ksplit(K / kGroup, ceil_div(N, kSlab) * M), (long long)ceil_div(N, kSlab), (long long)M);
         g_kernel_name = buf;
     } else {
         const SkConfig c = choose_gemm(M, K, N, with_workspace != 0);
-        g_kernel_name = w4a16_sk_name(c, 0, w4a16_sk_tiles(M, N, c) * c.splits);
+        g_kernel_name = w4a16_sk_name(c, kOne, w4a16_sk_tiles(M, N, c) * c.splits);
         if (!w4a16_sk_config_valid(M, K, N, c)) g_kernel_name += " NOT VALID";
     }
     return g_kernel_name.c_str();
 }
 
 const char* mcv_w4a16_parts_kernel_name(int64_t M, int64_t K, int64_t nslab, int n_parts, int gate_up) {
+    const int kind = gate_up ? kSilu : (n_parts == 1 ? kOne : kParts);
     if (M < 1 || K <= 0 || K % kGroup != 0 || nslab <= 0 || n_parts < 1 || n_parts > kMaxParts || (gate_up && n_parts != 2)) {
         g_kernel_name = "none (bad shape)";
-    } else if (w4a16_rows_pays(M, K, nslab, n_parts)) {
-        g_kernel_name = w4a16_rows_name(M, K, nslab, n_parts, gate_up != 0);
+    } else if (w4a16_rows_pays(M, K, nslab, kind)) {
+        g_kernel_name = w4a16_rows_name(M, K, nslab, kind);
     } else if (w4a16_parts_prefer_gemv(M, K, nslab, gate_up != 0)) {
         g_kernel_name = gate_up ? "w4a16_gate_up_silu_kernel" : "w4a16_gemv_multi_kernel";
     } else {
-        g_kernel_name = w4a16_sk_name(choose_gemm(M, K, (gate_up ? 2 : 1) * nslab * kSlab, false, true), gate_up ? 2 : 1, 0);
+        g_kernel_name = w4a16_sk_name(choose_gemm(M, K, (gate_up ? 2 : 1) * nslab * kSlab, false, true),
+                                      gate_up ? kSilu : kParts, 0);
     }
     return g_kernel_name.c_str();
 }

@@ -125,8 +125,6 @@ __device__ __forceinline__ int xcd_run(int b, int total) {
     return x * per + (x < rem ? x : rem) + i;
 }
 
-constexpr int kOne = 0, kParts = 1, kSilu = 2;
-
 template <int TM, int NWV, int NS, int KG, int KW, int WR, int EX>
 struct CfgS {
     static constexpr int WS = NWV / 2;                   // slabs per tile

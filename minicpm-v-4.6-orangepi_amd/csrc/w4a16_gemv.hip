@@ -600,7 +600,7 @@ int launch_w4a16_gemv(const void* x, int64_t M, int64_t K, int64_t N, const void
     W4Parts parts{};
     parts.count = 1;
     parts.p[0] = w4_part(qw, scales, zeros, zero_bias, N, out);
-    if (w4a16_rows_pays(M, K, nslab, 1) && w4a16_rows_ok(x, M, K, parts)) return launch_w4a16_rows(x, M, K, parts, stream);
+    if (w4a16_rows_pays(M, K, nslab, kOne) && w4a16_rows_ok(x, M, K, parts)) return launch_w4a16_rows(x, M, K, parts, stream);
     const GemvCfg cfg = choose_gemv(K / kGroup, nslab * M);
     auto fn = pick_kernel<kArgNone>(cfg.ksplit, cfg.gpw);
     hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>(nslab), static_cast<unsigned>(M)), dim3(64 * cfg.ksplit), 0,
@@ -850,7 +850,7 @@ int mcv_w4a16_gemv_multi(const void* x, int64_t M, int64_t K, const mcv_w4a16_pa
     // a few rows: each weight widened once for all of them; many: the GEMM
     // over the concatenated column tiles (both read x in 16-byte pieces)
     const hipStream_t st = static_cast<hipStream_t>(stream);
-    if (w4a16_rows_pays(M, K, total, n_parts) && w4a16_rows_ok(x, M, K, gp)) return launch_w4a16_rows(x, M, K, gp, st);
+    if (w4a16_rows_pays(M, K, total, n_parts == 1 ? kOne : kParts) && w4a16_rows_ok(x, M, K, gp)) return launch_w4a16_rows(x, M, K, gp, st);
     if (!w4a16_parts_prefer_gemv(M, K, total, false) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && w4a16_sk_fits(M, K, gp))
         return launch_w4a16_gemm_sk_parts(x, M, K, gp, nullptr, choose_gemm(M, K, total * kSlab, false, true), st);
     // The k-split the smallest part would get on its own (the decode shapes
@@ -879,14 +879,15 @@ int mcv_w4a16_gate_up_silu(const void* x, int64_t M, int64_t K, int64_t N, const
     if (M <= 0 || M > 65535) return fail(MCV_ERR_SHAPE, "mcv_w4a16_gate_up_silu: M must be in [1, 65535] (M=%lld)", (long long)M);
     if ((rc = require_device()) != MCV_OK) return rc;
     const int64_t nslab = ceil_div(N, kSlab);
-    // a few rows and many rows as mcv_w4a16_gemv_multi; the few-row rule is the
-    // single weight's, so gate and up round as two mcv_w4a16_gemv calls do
+    // a few rows and many rows as mcv_w4a16_gemv_multi; up to 32 rows the rule is the
+    // single weight's (but for its wide and its narrowest outputs), so gate and up
+    // round as two mcv_w4a16_gemv calls do
     W4Parts parts{};
     parts.count = 2;
     parts.p[0] = w4_part(qw_gate, scales_gate, zeros_gate, zero_bias_gate, N, act);
     parts.p[1] = w4_part(qw_up, scales_up, zeros_up, zero_bias_up, N, act);
     const hipStream_t st = static_cast<hipStream_t>(stream);
-    if (w4a16_rows_pays(M, K, nslab, 2) && w4a16_rows_ok(x, M, K, parts))
+    if (w4a16_rows_pays(M, K, nslab, kSilu) && w4a16_rows_ok(x, M, K, parts))
         return launch_w4a16_rows_silu(x, M, K, parts, act, st);
     if (!w4a16_parts_prefer_gemv(M, K, nslab, true) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && w4a16_sk_fits(M, K, parts))
         return launch_w4a16_gemm_sk_parts(x, M, K, parts, act, choose_gemm(M, K, 2 * nslab * kSlab, false, true), st);

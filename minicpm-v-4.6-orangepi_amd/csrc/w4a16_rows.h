@@ -42,9 +42,13 @@ __host__ __device__ constexpr uint32_t wide_zero_offset(int lane, int cb) {
 __host__ __device__ constexpr int wide_scale_base(int g, int Npad, int n0) { return (g * Npad + n0) * 2; }
 __host__ __device__ constexpr int wide_zero_base(int g, int Npad, int n0) { return (g * (Npad >> 3) + n0 / 8) * 4; }
 
+// What a launch computes: one weight's out = x . W; several weights' over the
+// same x; silu(x . gate) * (x . up).
+constexpr int kOne = 0, kParts = 1, kSilu = 2;
+
 // True where the few-row kernels are faster than the GEMV for M rows over `nslab`
-// slabs of `parts` weights.
-bool w4a16_rows_pays(int64_t M, int64_t K, int64_t nslab, int parts);
+// slabs in all (kSilu: of gate and of up each).
+bool w4a16_rows_pays(int64_t M, int64_t K, int64_t nslab, int kind);
 
 // True where the GEMM is faster than they are, on an output too large for the
 // GEMV (one weight).
@@ -62,8 +66,7 @@ int launch_w4a16_rows(const void* x, int64_t M, int64_t K, W4Parts parts, hipStr
 // the sums are launch_w4a16_rows' and round to fp16 before silu_mul_f16.
 int launch_w4a16_rows_silu(const void* x, int64_t M, int64_t K, W4Parts parts, void* act, hipStream_t stream);
 
-// The kernel's configuration for M x K over `nslab` slabs of `parts` weights
-// (`silu`: of gate and of up), as text.
-const char* w4a16_rows_name(int64_t M, int64_t K, int64_t nslab, int parts, bool silu);
+// The kernel's configuration for M x K over `nslab` slabs, as text.
+const char* w4a16_rows_name(int64_t M, int64_t K, int64_t nslab, int kind);
 
 }  // namespace mcv

@@ -469,16 +469,16 @@ bool w4a16_rows_ok(const void* x, int64_t M, int64_t K, const W4Parts& parts) {
 //   narrow weight (up to three slabs): K=1152 N=136 M=20 4.0 / 3.6.  Gate and up
 //   together do not (K=2048 N=136 M=32 5.0 / 5.8).
 // Past 32 rows only wide outputs.
-bool w4a16_rows_pays(int64_t M, int64_t K, int64_t nslab, int parts) {
+bool w4a16_rows_pays(int64_t M, int64_t K, int64_t nslab, int kind) {
     if (M < 2 || M > 64) return false;
     const int64_t G = K / kGroup, grid = M * nslab;
     if (G <= 2 && M <= 3) return false;
-    if (parts == 1 && rows_wide(M, K, nslab)) return true;
+    if (kind == kOne && rows_wide(M, K, nslab)) return true;
     if (M > 32) return false;
     if (G == 1) return grid > 4096;
-    if (G == 2) return grid > (parts == 1 ? 960 : 640);
+    if (G == 2) return grid > (kind == kParts ? 640 : 960);
     if (grid > 256) return (G != 4 || grid > 512) && (M > 16 || nslab <= 128 || grid * K > 500000);
-    if (M > 16) return parts == 1 && nslab < 4;
+    if (M > 16) return kind == kOne && nslab < 4;
     return nslab <= 64 && (K > 2048 || (G != 4 && G != 8 && nslab >= 32 && grid > 100));
 }
 
@@ -508,15 +508,15 @@ int launch_w4a16_rows_silu(const void* x, int64_t M, int64_t K, W4Parts parts, v
     return launch_any<true>(x, M, K, parts, act, stream);
 }
 
-const char* w4a16_rows_name(int64_t M, int64_t K, int64_t nslab, int parts, bool silu) {
+const char* w4a16_rows_name(int64_t M, int64_t K, int64_t nslab, int kind) {
     char buf[128];
-    if (parts == 1 && rows_wide(M, K, nslab)) {
+    if (kind == kOne && rows_wide(M, K, nslab)) {
         std::snprintf(buf, sizeof(buf), "w4a16_rows_wide_kernel<%d, %d, 2, 512>", M <= 16 ? 1 : (M <= 32 ? 2 : 4),
                       M > 32 && nslab >= 1536 ? 4 : 2);
     } else {
-        const RowsCfg c = choose_rows(M, K, nslab * kSlab, silu ? 2 : 1);
+        const RowsCfg c = choose_rows(M, K, nslab * kSlab, kind == kSilu ? 2 : 1);
         std::snprintf(buf, sizeof(buf), "w4a16_gemv_kernel_rows<%d, %d, %d, %s> (%lld workgroups of %d waves)", c.mb, c.cb,
-                      K / kGroup > c.ks && c.mb * c.cb <= 2 ? 2 : 1, silu ? "true" : "false", (long long)(nslab * 4 / c.cb),
+                      K / kGroup > c.ks && c.mb * c.cb <= 2 ? 2 : 1, kind == kSilu ? "true" : "false", (long long)(nslab * 4 / c.cb),
                       c.ks);
     }
     g_rows_name = buf;

@@ -546,3 +546,32 @@ def test_stream_handle_without_the_raw_query(mcv, monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
     monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
     assert mcv._stream() == 4711 and mcv._stream(SimpleNamespace(cuda_stream=5)) == 5
+
+
+def test_w4a16_parts_dispatch_builds(mcv):
+    """Every tile the dispatch picks for several weights and for gate + up is one
+    the library built; up to 32 rows gate + up never runs the GEMM."""
+    name, seen = mcv.lib().mcv_w4a16_parts_kernel_name, set()
+    for K in (128, 256, 384, 1024, 1152, 2048, 3584, 8192):
+        for nslab in (1, 3, 16, 40, 56, 80, 128, 300):
+            for M in (1, 8, 16, 33, 64, 96, 130, 200, 300, 512, 800, 1100, 2048, 8192):
+                for n_parts, gate_up in ((1, 0), (2, 0), (4, 0), (2, 1)):
+                    got = name(M, K, nslab, n_parts, gate_up).decode()
+                    assert "NOT BUILT" not in got and "none" not in got, (M, K, nslab, n_parts, gate_up, got)
+                    assert not (gate_up and M <= 32 and "gemm" in got)
+                    seen.add(got.split(" (")[0])
+    assert len([s for s in seen if "gemm_sk" in s]) == 11, seen
+    assert name(8, 100, 4, 2, 0) == name(8, 128, 4, 5, 0) == name(8, 128, 4, 3, 1) == b"none (bad shape)"
+
+
+def test_w4a16_gate_up_takes_the_gemv_sides_kernel(mcv):
+    """Where mcv_w4a16_gate_up_silu is documented bit-identical to two
+    mcv_w4a16_gemv calls, both run the few-row kernel or both the GEMV."""
+    name = mcv.lib().mcv_w4a16_parts_kernel_name
+    for K in list(range(128, 2305, 128)) + [2560, 3584, 3968, 4096, 8192]:
+        for M in range(1, 33):
+            for nslab in (1, 2, 3, 4, 8, 16, 17, 30, 32, 40, 56, 64, 65, 80, 96, 128, 129, 200, 399, 400, 799):
+                if M > 16 and not 4 <= nslab <= 399:
+                    continue
+                one, both = name(M, K, nslab, 1, 0).decode(), name(M, K, nslab, 2, 1).decode()
+                assert ("rows" in one) == ("rows" in both) and "wide" not in one, (M, K, nslab, one, both)

@@ -664,3 +664,59 @@ def test_gemm_two_stage_tiles(mcv, oracle, cuda, M, K, N, tm):
     torch.cuda.synchronize()
     ref = oracle.w4a16_matmul(x, oracle.unpack_awq(qweight, qzeros), scales)
     _check(_host_f32(out), ref, f"tm={tm} M={M} K={K} N={N}")
+
+
+# Gate + up over the rows and widths that run the GEMV, and the few-row kernel with
+# one and two 16-row blocks: two GEMV-side calls and silu_mul, bit for bit.
+@pytest.mark.parametrize("M,K,N", [(5, 1024, 3584), (16, 1024, 3584), (16, 3584, 520), (2, 1024, 3584), (17, 1024, 520),
+                                   (24, 256, 2048), (32, 1024, 3584), (32, 512, 1000), (32, 3584, 264), (20, 384, 6144),
+                                   (12, 256, 4096)], ids=lambda v: str(v))
+def test_gate_up_silu_bits_at_several_rows(mcv, cuda, M, K, N):
+    torch = _torch()
+    rng = np.random.default_rng(70 + M + K + N)
+    wg, wu = (_dev_weight(mcv, *synth_w4a16(rng, K, N)[1:]) for _ in range(2))
+    xd = _to_dev(f16_normal(rng, (M, K), 1.0))
+    fused = mcv.mlp_gate_up_silu_w4a16(xd, wg, wu)
+    three = mcv.silu_mul(mcv.matmul_w4a16_gemv(xd, wg), mcv.matmul_w4a16_gemv(xd, wu))
+    assert torch.equal(fused.view(torch.int16), three.view(torch.int16))
+
+
+# Every tile that the dispatch takes for several weights and for gate + up: K of
+# three and five groups (one k-part) and of six to eight (two), row and column
+# remainders, a part boundary inside the columns.
+PARTS_TILES = [("32, 2, 3, 1, 1, 1", 257, 384, (136, 40), 77, 424), ("32, 2, 3, 2, 2, 1", 385, 768, (64, 8), 33, 680),
+               ("32, 4, 3, 1, 1, 1", 65, 384, (3000, 2440), 65, 2712), ("32, 4, 3, 2, 2, 1", 65, 1024, (2056, 3384), 65, 2712),
+               ("64, 2, 3, 1, 1, 1", 97, 384, (2000, 2104), 33, 4104), ("64, 2, 3, 2, 2, 1", 97, 768, (4040, 72), 33, 4104),
+               ("64, 4, 3, 1, 1, 1", 129, 384, (6000, 536), 65, 5464), ("64, 4, 3, 2, 2, 1", 129, 1024, (72, 6456), 65, 5464),
+               ("64, 4, 2, 1, 1, 1", 520, 384, (3144, 3400), 257, 5464), ("128, 4, 3, 1, 1, 0", 257, 384, (3144, 4040), 129, 6552),
+               ("128, 4, 2, 1, 1, 1", 769, 384, (3720, 3848), 385, 7000)]
+
+
+@pytest.mark.parametrize("tile,M,K,Ns,Mg,Ng", PARTS_TILES, ids=lambda v: str(v).replace(", ", "_"))
+def test_parts_every_tile(mcv, oracle, cuda, tile, M, K, Ns, Mg, Ng):
+    torch = _torch()
+    name = mcv.lib().mcv_w4a16_parts_kernel_name
+    slabs = sum(-(-n // 64) for n in Ns)
+    assert f"sk_kernel<{tile}>" in name(M, K, slabs, len(Ns), 0).decode()
+    assert f"sk_kernel<{tile}>" in name(Mg, K, -(-Ng // 64), 2, 1).decode()
+    rng = np.random.default_rng(M + K + sum(Ns))
+    x = f16_normal(rng, (max(M, Mg), K), 1.0)
+    xf = torch.from_numpy(x.view(np.float16)).cuda().double()
+
+    def weight(N, zb):
+        _, qw, qz, sc = synth_w4a16(rng, K, N)
+        w = _dev_weight(mcv, qw, qz, sc)
+        w = mcv.W4A16QuantizedWeight(w.qweight, w.scales, w.zeros, K, N, zb)
+        vals = (oracle.unpack_awq(qw, qz) - np.int8(zb)).astype(np.float64) * \
+            np.repeat(sc.view(np.float16).astype(np.float64), 128, axis=0)
+        return w, torch.from_numpy(vals).cuda()
+
+    parts = [weight(N, i & 1) for i, N in enumerate(Ns)]
+    for o, (w, wf) in zip(mcv.matmul_w4a16_multi(_to_dev(x[:M]), [w for w, _ in parts]), parts):
+        # fp32 sums of K exact products, one rounding of the output
+        ref, mag = xf[:M] @ wf, xf[:M].abs() @ wf.abs()
+        assert bool(((o.double() - ref).abs() <= 2.0 ** -11 * ref.abs() + K * 2.0 ** -24 * mag + 2.0 ** -24).all())
+    (wg, gf), (wu, uf) = weight(Ng, 1), weight(Ng, 0)
+    act = _host_f32(mcv.mlp_gate_up_silu_w4a16(_to_dev(x[:Mg]), wg, wu))
+    g, u = ((xf[:Mg] @ f).half().cpu().view(torch.int16).numpy().view(np.uint16) for f in (gf, uf))
+    _check(act, oracle.silu_mul(g, u).view(np.float16).astype(np.float32), f"gate_up {tile}")
