@@ -155,9 +155,11 @@ int mcv_w4a16_unpack_host(const void* qw_host, const uint16_t* scales_host,
 /* out[M][N] fp16 = x[M][K] fp16 . dequant(W) with fp32 accumulation.
  * Replaces matmul_w4a16 / aclnnMatmulW4a16Custom (src/csrc/lib/ops.cpp:1030-1095,
  * kernel src/csrc/custom_ops/op_kernel/matmul_w4a16_custom.cpp:157-168), which
- * accepts M = 1 only; any M >= 1 is accepted here.  Small M runs the streaming
- * GEMV kernel, larger M the LDS-dequant fp16 MFMA GEMM, unsplit (without a
- * workspace it never splits K; mcv_w4a16_gemm_ws may). */
+ * accepts M = 1 only; any M >= 1 is accepted here.  One row runs the streaming
+ * GEMV kernel, a few rows the few-row MFMA kernels (2 to 32 rows, 64 over a
+ * vocabulary), larger M the tiled fp16 MFMA GEMM, unsplit (without a workspace
+ * it never splits K; mcv_w4a16_gemm_ws may); which of them is a matter of M, K
+ * and N (mcv_w4a16_gemm_kernel_name). */
 int mcv_w4a16_gemm(const void* x_dev, int64_t M, int64_t K, int64_t N,
                    const void* qw_dev, const void* scales_dev, const void* zeros_dev,
                    int zero_bias, void* out_dev, mcv_stream_t stream);

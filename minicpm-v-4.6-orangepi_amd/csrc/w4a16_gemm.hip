@@ -1,10 +1,11 @@
 // w4a16_gemm.hip -- the W4A16 matmul dispatch for any M, gfx950.
 //
-// out[M][N] = x[M][K] . W[K][N], W in the slab-64 int4 layout.  Decode-sized
-// M streams the weights through the GEMV (w4a16_gemv.hip), one grid row per
-// activation row; larger M runs the half-slab MFMA GEMM (w4a16_gemm_sk.hip),
-// which reuses each widened weight operand across TM rows, in the tile shape
-// and K split picked here.
+// out[M][N] = x[M][K] . W[K][N], W in the slab-64 int4 layout.  One row streams
+// the weights through the GEMV (w4a16_gemv.hip; one grid row per activation row
+// where a few rows of a small weight are as fast that way); a few rows run the
+// kernels that widen every weight once for all of them (w4a16_rows.hip); larger M
+// runs the half-slab MFMA GEMM (w4a16_gemm_sk.hip), which reuses each widened
+// weight operand across TM rows, in the tile shape and K split picked here.
 //
 // The reference has no M > 1 quantised path: its matmul_w4a16 is M = 1 only
 // (src/csrc/lib/ops.cpp:1030-1095) and its prefill runs dense fp16 aclnnMm
@@ -58,7 +59,7 @@ bool small_output(int64_t M, int64_t N) { return M >= 1 && (M < 8 || M * N < 655
 // M=512 K=1024 N=3584 64x128 two k-parts 8.3-8.5 (32x64 10.0-11.6); M=512
 // K=3584 N=1024 32x64 two k-parts 10.1 (32x128 split 2 ways 11.4-12.1, 64x64
 // split 2 ways 10.8); M=128 K=1024 N=3584 32x64 two k-parts 5.5 (one k-part
-// 6.6, 32x128 6.7-7.0); M=128 K=3584 N=1024 32x64 split 2 ways, two k-parts
+// 6.6, 32x128 6.7-7.0); M=128 K=3584 N=1024 32x64 split 4 ways, two k-parts
 // 7.96 (3 ways 7.93, 2 ways 8.8; one k-part 4 ways 9.7; 32x128 split 4 ways
 // 9.6-9.8); M=64 K=3584 N=1024 32x64 split 4 ways 7.2 (3 ways 7.4, 8 ways
 // 8.0); M=128 K=2048 N=1024 2 ways 7.1 (3 ways 6.85); 64x64 two
